@@ -120,7 +120,7 @@ def _positions(case, seed):
         w = _torus(case["voxels"])
         return w["V"] + rng.uniform(-0.08, 0.08, size=w["V"].shape) * w["edge"][:, None]
     V, _, _ = _grid(case["n"])
-    return V + rng.normal(0.0, 0.12 * 2.0 / case["n"], size=V.shape)
+    return V + rng.normal(0.0, 0.08 * 2.0 / case["n"], size=V.shape)
 
 
 def _planes(case, seed, ids):
@@ -695,12 +695,15 @@ def _project_lines(SV, curves, of, P):
         if m.numel() == 0:
             continue
         a = SV[torch.as_tensor(np.asarray(curve), device=P.device)]
-        e = torch.roll(a, -1, 0) - a
+        b = torch.roll(a, -1, 0)
+        e = b - a
         q = P[m][:, None, :] - a
-        t = ((q * e).sum(-1) / (e * e).sum(-1)).clamp(0, 1)
-        j = ((q - t[..., None] * e) ** 2).sum(-1).argmin(dim=1)
+        t = ((q * e).sum(-1) / (e * e).sum(-1))[..., None]
+        pt = torch.where(t <= 0, a, torch.where(t >= 1, b, a + t * e))
+        # the nearer one, of two that share the nearest end the first
+        j = ((P[m][:, None, :] - pt) ** 2).sum(-1).argmin(dim=1)
         r = torch.arange(m.numel(), device=P.device)
-        O[m], T[m] = a[j] + t[r, j][:, None] * e[j], e[j] / e[j].norm(dim=1, keepdim=True)
+        O[m], T[m] = pt[r, j], e[j] / e[j].norm(dim=1, keepdim=True)
     return O, T
 
 
