@@ -59,6 +59,7 @@ struct hexopt_ctx {
   DevBuf d_conn, d_tile_hex, d_tile_col, d_tile_lv, d_lv_gid, d_lv_slot, d_lv_first, d_lidx, d_tile_corner, d_sv_gid,
       d_sv_off, d_sv_slots, d_lv_dst, d_v_dst;
   DevBuf d_iso;  // vertices without hexes
+  DevBuf d_vperm, d_rows;  // caller's id of every vertex; rows in the caller's order, in transit
   DevBuf d_torder;       // plane queries sorted by vertex (Morton) order
   DevBuf d_cgsave;       // CG state of the last direction solve, read back with the line search
   int n_iso = 0;
@@ -123,15 +124,39 @@ int upload(hexopt_ctx* c, DevBuf& b, const std::vector<T>& v) {
   return HEXOPT_OK;
 }
 
-// caller rows (nV x 3) -> SoA Morton order
-void to_soa(const MeshLayout& L, const double* V, std::vector<double>& out) {
-  out.resize((size_t)3 * L.nV);
-  for (int i = 0; i < L.nV; ++i)
-    for (int d = 0; d < 3; ++d) out[(size_t)d * L.nV + i] = V[(size_t)L.vperm[i] * 3 + d];
+// The context's device for the calls in this scope, whatever the calling thread's is (a kernel
+// needs its stream's device current; copies do not)
+struct OnDevice {
+  int before = -1;
+  explicit OnDevice(int device) {
+    if (hipGetDevice(&before) != hipSuccess || before == device || hipSetDevice(device) != hipSuccess) before = -1;
+  }
+  ~OnDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
+// caller rows (nV x 3, host) -> a field of this numbering on the device, queued on the stream.
+// The staging buffer is the context's: its uses follow one another on the one stream.
+int rows_in(hexopt_ctx* c, int prec, const void* rows, void* field) {
+  const OnDevice on(c->device);
+  const size_t bytes = (size_t)3 * c->L.nV * (prec / 8);
+  HIPCHK(c, c->d_rows.ensure(bytes));
+  HIPCHK(c, hipMemcpyAsync(c->d_rows.p, rows, bytes, hipMemcpyHostToDevice, c->stream));
+  launch_rows_to_fields(prec, c->L.nV, c->d_vperm.as<int>(), c->d_rows.p, field, c->stream);
+  HIPCHK(c, hipGetLastError());
+  return HEXOPT_OK;
 }
-void from_soa(const MeshLayout& L, const double* S, double* V) {
-  for (int i = 0; i < L.nV; ++i)
-    for (int d = 0; d < 3; ++d) V[(size_t)L.vperm[i] * 3 + d] = S[(size_t)d * L.nV + i];
+// and back; waits for the stream
+int rows_out(hexopt_ctx* c, int prec, const void* field, void* rows) {
+  const OnDevice on(c->device);
+  const size_t bytes = (size_t)3 * c->L.nV * (prec / 8);
+  HIPCHK(c, c->d_rows.ensure(bytes));
+  launch_fields_to_rows(prec, c->L.nV, c->d_vperm.as<int>(), field, c->d_rows.p, c->stream);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipMemcpyAsync(rows, c->d_rows.p, bytes, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return HEXOPT_OK;
 }
 
 int nblocks(long n) { long b = (n + 255) / 256; if (b < 1) b = 1; if (b > 2048) b = 2048; return (int)b; }
@@ -237,10 +262,12 @@ hexopt_ctx* hexopt_create(int nV, const double* V, int nH, const int32_t* hexes,
     c->n_iso = (int)iso.size();
     rc |= upload(c, c->d_iso, iso);
   }
-  std::vector<double> soa;
-  to_soa(L, V, soa);
-  rc |= upload(c, c->d_rest, soa);
-  rc |= upload(c, c->d_cur, soa);
+  rc |= upload(c, c->d_vperm, L.vperm);
+  const size_t xb = (size_t)3 * L.nV * sizeof(double);
+  if (c->d_rest.ensure(xb) != hipSuccess || c->d_cur.ensure(xb) != hipSuccess) rc = HEXOPT_EHIP;
+  if (rc == HEXOPT_OK) rc |= rows_in(c, 64, V, c->d_rest.p);
+  if (rc == HEXOPT_OK && hipMemcpyAsync(c->d_cur.p, c->d_rest.p, xb, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+    rc = HEXOPT_EHIP;
   if (rc != HEXOPT_OK || hipStreamSynchronize(c->stream) != hipSuccess) {
     g_create_error = "device upload failed: " + c->err;
     hexopt_destroy(c);
@@ -272,22 +299,15 @@ const char* hexopt_last_error(hexopt_ctx* c) { return c ? c->err.c_str() : "null
 
 int hexopt_set_positions(hexopt_ctx* c, int which, const double* V) {
   if (!c || !V || (which != HEXOPT_REST && which != HEXOPT_CURRENT)) return HEXOPT_EINVAL;
-  std::vector<double> soa;
-  to_soa(c->L, V, soa);
-  DevBuf& b = which == HEXOPT_REST ? c->d_rest : c->d_cur;
-  HIPCHK(c, hipMemcpyAsync(b.p, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  const int rc = rows_in(c, 64, V, (which == HEXOPT_REST ? c->d_rest : c->d_cur).p);
+  if (rc) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return HEXOPT_OK;
 }
 
 int hexopt_get_positions(hexopt_ctx* c, int which, double* V) {
   if (!c || !V || (which != HEXOPT_REST && which != HEXOPT_CURRENT)) return HEXOPT_EINVAL;
-  std::vector<double> soa((size_t)3 * c->L.nV);
-  DevBuf& b = which == HEXOPT_REST ? c->d_rest : c->d_cur;
-  HIPCHK(c, hipMemcpyAsync(soa.data(), b.p, soa.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  from_soa(c->L, soa.data(), V);
-  return HEXOPT_OK;
+  return rows_out(c, 64, (which == HEXOPT_REST ? c->d_rest : c->d_cur).p, V);
 }
 
 int hexopt_copy_positions(hexopt_ctx* c, int from, int to) {
@@ -1726,31 +1746,9 @@ static int adj_common(hexopt_ctx* c, int precision, const void* X, const void* v
   HIPCHK(c, c->d_G.ensure((size_t)3 * nV * es));
   HIPCHK(c, c->d_v.ensure((size_t)3 * nV * es));
   HIPCHK(c, c->d_halo.ensure((size_t)6 * (c->L.nSlots + 1) * sizeof(double)));
-  auto soa = [&](const void* src, DevBuf& dst) -> int {
-    std::vector<unsigned char> tmp((size_t)3 * nV * es);
-    for (int i = 0; i < nV; ++i)
-      for (int d = 0; d < 3; ++d)
-        std::memcpy(&tmp[((size_t)d * nV + i) * es], (const unsigned char*)src + ((size_t)c->L.vperm[i] * 3 + d) * es, es);
-    HIPCHK(c, hipMemcpyAsync(dst.p, tmp.data(), tmp.size(), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return HEXOPT_OK;
-  };
-  int rc = soa(X, c->d_X);
-  if (rc) return rc;
-  if (v) rc = soa(v, c->d_v);
+  int rc = rows_in(c, precision, X, c->d_X.p);
+  if (rc == HEXOPT_OK && v) rc = rows_in(c, precision, v, c->d_v.p);
   return rc;
-}
-
-static int adj_out(hexopt_ctx* c, int precision, void* out) {
-  const size_t es = precision == 64 ? 8 : 4;
-  const int nV = c->L.nV;
-  std::vector<unsigned char> tmp((size_t)3 * nV * es);
-  HIPCHK(c, hipMemcpyAsync(tmp.data(), c->d_G.p, tmp.size(), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int i = 0; i < nV; ++i)
-    for (int d = 0; d < 3; ++d)
-      std::memcpy((unsigned char*)out + ((size_t)c->L.vperm[i] * 3 + d) * es, &tmp[((size_t)d * nV + i) * es], es);
-  return HEXOPT_OK;
 }
 
 int hexopt_energy_grad(hexopt_ctx* c, const hexopt_params* prm, int precision, const void* X, const double* aL, void* G) {
@@ -1767,7 +1765,7 @@ int hexopt_energy_grad(hexopt_ctx* c, const hexopt_params* prm, int precision, c
   SoftDev sd = soft_with(c, prm);
   launch_grad(precision, c->tm, refop(c), c->d_X.p, c->d_G.p, tet_mass(prm), sd, d_aL, c->d_halo.p, c->stream);
   HIPCHK(c, hipGetLastError());
-  return adj_out(c, precision, G);
+  return rows_out(c, precision, c->d_G.p, G);
 }
 
 int hexopt_hvp(hexopt_ctx* c, const hexopt_params* prm, int precision, const void* X, const void* v, void* Hv) {
@@ -1779,7 +1777,7 @@ int hexopt_hvp(hexopt_ctx* c, const hexopt_params* prm, int precision, const voi
   SoftDev sd = soft_with(c, prm);
   launch_hvp(precision, c->tm, refop(c), c->d_X.p, c->d_v.p, c->d_G.p, tet_mass(prm), sd, c->d_halo.p, c->stream);
   HIPCHK(c, hipGetLastError());
-  return adj_out(c, precision, Hv);
+  return rows_out(c, precision, c->d_G.p, Hv);
 }
 
 int hexopt_scaled_jacobian(hexopt_ctx* c, int which, double* min_j, double* avg_j, double* per_hex) {

@@ -61,6 +61,10 @@ struct SoftDev {
   const uint8_t* fixed;
 };
 
+// rows (n x 3, the caller's order) <-> fields f[d*n + i] with vertex i the caller's perm[i];
+// prec 64: double, else float
+void launch_rows_to_fields(int prec, int n, const int* perm, const void* rows, void* f, hipStream_t st);
+void launch_fields_to_rows(int prec, int n, const int* perm, const void* f, void* rows, hipStream_t st);
 void launch_ref_cube(const double* X, int nV, const int* conn, int nH, const uint8_t* hflag, int cube, double* invs,
                      int* n_general, hipStream_t st);
 void launch_ref_general(const double* X, int nV, const int* conn, int nH, const uint8_t* hflag, int cube, double* B,
