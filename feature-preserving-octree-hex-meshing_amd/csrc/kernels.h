@@ -23,6 +23,7 @@ struct TileMesh {
   const uint8_t* tile_corner;
   const int* lv_dst;  // per local vertex: place among all (tile, vertex) pairs, vertex by vertex
   const int* v_dst;   // nV+1: each vertex's run of places
+  int nPairs;         // number of those pairs
 };
 
 enum RefMode { REF_CUBE = 0, REF_GENERAL = 1 };
@@ -111,17 +112,9 @@ void launch_hvp(int prec, const TileMesh& tm, const RefOp& ro, const void* X, co
 // FP32 optimiser (adjoint formulation of the SLIM step)
 void launch_adj_local32(const TileMesh& tm, const RefOp& ro, const double* X, float* K, double M, double prox,
                         const SoftDev& sd, float* rhs, float* invd, float* halo, int* n_inverted, hipStream_t st);
-void launch_apply32(const TileMesh& tm, const RefOp& ro, const float* K, const float* p, float* out, double prox,
-                    const SoftDev& sd, float* halo, double* part_tile, double* part_fix, double* part_line,
-                    hipStream_t st);
 void launch_apply32_f64(const TileMesh& tm, const RefOp& ro, const float* K, const float* p, double* out, double prox,
                         const SoftDev& sd, double* halo, hipStream_t st);
-void launch_cg_init32(int n, const float* rhs, const float* tmp, float* r, double* pb, double* pr, int nb, void* state,
-                      const float* invd, float* p, double* pabs, double tol, hipStream_t st);
-void launch_cg_update32(int n, void* state, float* x, float* r, float* z, const float* p, const float* tmp,
-                        const float* invd, double* prr, double* prz, int nb, float* p_out, hipStream_t st);
-void launch_cg_zero_if32(int n, void* state, float* x, int nb, hipStream_t st);
-// Fused FP32 CG (Eigen's algorithm, FP64 dot products) on the CG operator of launch_apply32:
+// Fused FP32 CG (Eigen's algorithm, FP64 dot products) on the CG operator:
 // launch_cg32_init sets x = 0, r = b, z = b / diag, p_prev = 0 and the state; each
 // launch_cg32_iteration is one CG iteration reading z and p_prev, writing p_new and the
 // updated x, r, z (zout may alias z); k is the CG iteration and last marks the final one (the
@@ -153,8 +146,20 @@ void launch_cg32_iteration(const TileMesh& tm, const RefOp& ro, const float* K, 
                            float* out, float* halo, const float* invd, float* x, float* r, float* zout, void* state,
                            double* part_tile, double* part_rr, double* part_rz, double* part_qz, double* part_bzq,
                            double* part_qq, int k, int last, hipStream_t st);
-void launch_residual64(int n, const float* b, const double* Ld, float* r32, double* part, int nb, double* out,
-                       hipStream_t st);
+// FP64 CG (Eigen's algorithm with its Jacobi preconditioner) on L x = rhs from x = cur, a_L = 0:
+// the solution goes to x, both vectors with 3 nV + nL entries. out: the a_L rows of the product;
+// halo: 3 * nPairs values; part: 8 arrays of partials; sd without glue.
+struct Cg64 {
+  double *x, *r, *z, *p[2], *out, *halo;
+  void* state;
+  double* part[8];
+};
+void launch_cg64(const TileMesh& tm, const RefOp& ro, const double* K, double prox, const SoftDev& sd, const int* iso,
+                 int niso, const double* cur, const double* rhs, const double* invd, const Cg64& w, int iters,
+                 double tol, hipStream_t st);
+// its operator pass alone (the one that forms the first residual)
+void launch_cg64_operator(const TileMesh& tm, const RefOp& ro, const double* K, const SoftDev& sd, const double* cur,
+                          const Cg64& w, hipStream_t st);
 void launch_f2d(int n, const float* a, double* b, hipStream_t st);
 void launch_d2f(int n, const double* a, float* b, hipStream_t st);
 // b = -g / 2 on the vertex rows of g (the FP64 adjoint gradient, in place) and the a_L rows at
