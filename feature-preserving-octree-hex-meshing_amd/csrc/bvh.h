@@ -43,7 +43,7 @@ struct SurfaceDev {
 constexpr int kBvhBlock = 128;
 constexpr int kBvhMaxDepth = 48;
 // traversal stack entries per lane for a tree of `depth` levels (root = level 1): a
-// depth-first walk holds at most one frame per level, plus one spare; never above
+// depth-first walk holds at most one waiting child per level, plus spares; never above
 // kBvhMaxDepth + 2 (surfaces with deeper trees are refused at creation)
 __host__ __device__ inline int stack_frames(int depth) {
   const int d = depth < 1 ? 1 : depth;
@@ -58,14 +58,18 @@ __host__ __device__ inline int stack_frames(int depth) {
 void launch_closest(const SurfaceDev& s, int nq, const double* P, int soa, int stride, const int* ids, double* S, int* I,
                     double* C, double* N, double* sqrD, int* status, hipStream_t st, const int* order = nullptr);
 
+// Lanes of a wave that take a query each, for nq queries in a launch: a block of kBvhBlock
+// threads takes closest_lanes(nq) * kBvhBlock / 64 of them.
+int closest_lanes(int nq);
+
 // Several surfaces in one launch: segment j's queries are order[q0 .. q0 + n) against surface
-// s, taken by blocks block0 .. block0 + ceil(n / kBvhBlock) (segments in increasing block0,
+// s, taken by blocks block0 .. block0 + ceil(n / a block's queries) (segments in increasing block0,
 // the first at block 0). Writes C and N (indexed by the query, as launch_closest does).
 struct PatchSeg {
   SurfaceDev s;
   int block0, q0, n, pad;
 };
-void launch_closest_segs(const PatchSeg* segs, int nseg, int nblocks, int max_depth, const double* P, int soa,
+void launch_closest_segs(const PatchSeg* segs, int nseg, int nblocks, int lanes, int max_depth, const double* P, int soa,
                          int stride, const int* ids, const int* order, double* C, double* N, int* status,
                          hipStream_t st);
 

@@ -5,8 +5,10 @@
 // (AABB.cpp:364-441) exactly -- visit a child whose box contains the point, then the nearer
 // child (by exterior box distance) and then the other, each only while it can still beat the
 // current best, leaves compared with a strict '<' (set_min, AABB.cpp:735-779) -- so the face
-// chosen on ties is the reference's. The recursion becomes an explicit stack of packed
-// frames (node | visit state | visited-children bits) that lives in LDS, one column per lane.
+// chosen on ties is the reference's. At a node that order is settled on arrival: a child that
+// contains the point is entered whatever the best is, the left one first; any other child after
+// those, the nearer first, if its box distance is below the best at that moment. So one child is
+// entered at once and the other waits on a stack with its box distance; no node is visited twice.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include "bvh.h"
@@ -84,26 +86,41 @@ __device__ __forceinline__ void load3(const double* V, int i, double o[3]) {
   o[0] = V[(size_t)i * 3]; o[1] = V[(size_t)i * 3 + 1]; o[2] = V[(size_t)i * 3 + 2];
 }
 
-// frame packing: node (26 bits) | state (3 bits) << 26 | visited (2 bits) << 29
-__device__ __forceinline__ int fr_node(unsigned f) { return (int)(f & 0x3ffffffu); }
-__device__ __forceinline__ unsigned fr_state(unsigned f) { return (f >> 26) & 7u; }
-__device__ __forceinline__ unsigned fr_seen(unsigned f) { return (f >> 29) & 3u; }
-__device__ __forceinline__ unsigned fr_make(int n, unsigned st, unsigned seen) { return (unsigned)n | (st << 26) | (seen << 29); }
+// Box distance of a waiting child, kept as the float at or below it: half the stack that exact
+// distances would take. It decides against `best` except within a float's spacing of it (and
+// below the float range), where the distance is taken again from the child's box.
+__device__ __forceinline__ float key_below(double d) {
+  float k = (float)d;
+  if ((double)k > d) k = __int_as_float(__float_as_int(k) - 1);
+  return k;
+}
+__device__ __forceinline__ bool key_beats(float k, double best, const double* __restrict__ box, const double p[3]) {
+  if (k < 0.0f) return true;  // contains the point
+  if ((double)k >= best) return false;
+  if (k > 1e-37f && (double)__int_as_float(__float_as_int(k) + 1) < best) return true;
+  return box_ext_dist(box, p) < best;
+}
 
-// six waves per SIMD (80 registers, 2 values spilled) instead of the five that 82 registers
-// leave: more walks in flight to cover the dependent node fetches (the four patch walks of the
-// 1.1M-hex torus refresh: 275-279 against 294-295 us; eight waves with 33 spills, 284-287)
-__global__ __launch_bounds__(kBvhBlock) __attribute__((amdgpu_waves_per_eu(6))) void closest_kernel(SurfaceDev s0, const PatchSeg* __restrict__ segs, int nseg,
+// Latency- and issue-bound: per step one record of 128 bytes at a place that the step before
+// chose, two box distances or a point-triangle distance in FP64. 24,578 queries on 20,480
+// triangles: 452 us with a stack of frames that were come back to after each child (and their
+// records fetched again), 245 us with waiting children; the four patch walks of the 1.1M-hex torus
+// (411,080 queries) 306 -> 253 us. A leaf with one division for all its regions instead of a
+// branch each: 294 us; inner steps alone until every lane stands at a leaf: 682 us.
+__global__ __launch_bounds__(kBvhBlock) void closest_kernel(SurfaceDev s0, const PatchSeg* __restrict__ segs, int nseg, int lanes,
                                                             int nq, const double* P, int soa, int stride,
                                                             const int* ids, const int* order, double* S, int* I,
                                                             double* Cout, double* Nout, double* sqrDout, int* status) {
-  // one frame per tree level: (depth + 1) x kBvhBlock entries of dynamic LDS (see
+  // one waiting child per tree level: stack_frames(depth) x kBvhBlock entries of dynamic LDS (see
   // launch_closest), so shallow trees leave room for more resident blocks
-  extern __shared__ unsigned stack[];
+  extern __shared__ uint2 stack[];
   // with segments, each block belongs to one (the last segment starting at or before it) and
   // walks that segment's tree for that segment's queries; the choice is the same in every lane
   SurfaceDev s = s0;
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
+  // `lanes` of a wave's 64 lanes take a query each (closest_lanes)
+  if ((int)(threadIdx.x & 63) >= lanes) return;
+  const int per_block = lanes * (kBvhBlock / 64), in_block = (threadIdx.x >> 6) * lanes + (threadIdx.x & 63);
+  int k = blockIdx.x * per_block + in_block;
   if (nseg > 0) {
     int lo = 0, hi = nseg - 1;
     while (lo < hi) {
@@ -112,7 +129,7 @@ __global__ __launch_bounds__(kBvhBlock) __attribute__((amdgpu_waves_per_eu(6))) 
       else hi = mid - 1;
     }
     s = segs[lo].s;
-    const int local = ((int)blockIdx.x - segs[lo].block0) * blockDim.x + threadIdx.x;
+    const int local = ((int)blockIdx.x - segs[lo].block0) * per_block + in_block;
     if (local >= segs[lo].n) return;
     k = segs[lo].q0 + local;
   } else if (k >= nq) {
@@ -127,64 +144,50 @@ __global__ __launch_bounds__(kBvhBlock) __attribute__((amdgpu_waves_per_eu(6))) 
   } else {
     load3(P, pi, p);
   }
-  unsigned* stk = stack + threadIdx.x;  // column per lane: entry k at stk[k*kBvhBlock]
-  int top = 0;
+  uint2* stk = stack + threadIdx.x;  // column per lane: (node, key) k at stk[k*kBvhBlock]
+  int top = 0, n = 0;
   double best = INFINITY;
   int bf = -1;
   double bc[3] = {0, 0, 0};
-  stk[0] = fr_make(0, 0, 0);
-  top = 1;
   bool overflow = false;
-  while (top > 0) {
-    unsigned f = stk[(top - 1) * kBvhBlock];
-    const int n = fr_node(f);
+  for (;;) {
     // the node's record in one go: children's boxes (inner) or the face's corners (leaf)
     const double2* r2 = reinterpret_cast<const double2*>(s.rec + (size_t)n * kNodeRec);
     double x[12];
 #pragma unroll
     for (int j = 0; j < 6; ++j) { const double2 v = r2[j]; x[2 * j] = v.x; x[2 * j + 1] = v.y; }
     const int4 w = reinterpret_cast<const int4*>(r2)[6];
-    const int pr = w.z;
-    if (pr >= 0) {  // leaf_squared_distance + set_min
+    bool down = false;  // enter node n next; else the next waiting child
+    if (w.z >= 0) {  // leaf_squared_distance + set_min
       const double a[3] = {x[0], x[1], x[2]}, b[3] = {x[3], x[4], x[5]}, c[3] = {x[6], x[7], x[8]};
       double r[3];
       closest_on_tri(p, a, b, c, r);
       // (p - c).squaredNorm() in Eigen's order
       const double d = (p[0] - r[0]) * (p[0] - r[0]) + ((p[1] - r[1]) * (p[1] - r[1]) + (p[2] - r[2]) * (p[2] - r[2]));
-      if (d < best) { best = d; bf = pr; bc[0] = r[0]; bc[1] = r[1]; bc[2] = r[2]; }
-      --top;
-      continue;
-    }
-    const int L = w.x, R = w.y;
-    const double* bl = x;
-    const double* br = x + 6;
-    unsigned state = fr_state(f), seen = fr_seen(f);
-    int child = -1;
-    while (child < 0 && state < 4) {
-      if (state == 0) {                         // must look left if in box
-        state = 1;
-        if (box_contains(bl, p)) { seen |= 1; child = L; }
-      } else if (state == 1) {                  // must look right if in box
-        state = 2;
-        if (box_contains(br, p)) { seen |= 2; child = R; }
-      } else {                                  // then nearer first, each only if it can win
-        const double lm = box_ext_dist(bl, p), rm = box_ext_dist(br, p);
-        const bool left_first = lm < rm;
-        const bool first = state == 2;
-        state += 1;
-        const bool take_left = left_first == first;
-        if (take_left) {
-          if (!(seen & 1) && lm < best) { seen |= 1; child = L; }
-        } else {
-          if (!(seen & 2) && rm < best) { seen |= 2; child = R; }
-        }
+      if (d < best) { best = d; bf = w.z; bc[0] = r[0]; bc[1] = r[1]; bc[2] = r[2]; }
+    } else {
+      const bool cl = box_contains(x, p), cr = box_contains(x + 6, p);
+      const double lm = box_ext_dist(x, p), rm = box_ext_dist(x + 6, p);
+      const bool left = cl || (!cr && lm < rm);  // which child comes first
+      n = left ? w.x : w.y;
+      down = cl || cr || (left ? lm : rm) < best;
+      // best only falls, so a child that cannot beat it now need not wait
+      const double d2 = left ? rm : lm;
+      const bool both = cl && cr;
+      if (both || d2 < best) {
+        if (top >= cap) { overflow = true; break; }
+        stk[top * kBvhBlock] = make_uint2((unsigned)(left ? w.y : w.x),
+                                          (unsigned)__float_as_int(both ? -1.0f : key_below(d2)));
+        ++top;
       }
     }
-    if (child < 0) { --top; continue; }
-    stk[(top - 1) * kBvhBlock] = fr_make(n, state, seen);
-    if (top >= cap) { overflow = true; break; }
-    stk[top * kBvhBlock] = fr_make(child, 0, 0);
-    ++top;
+    while (!down && top > 0) {
+      --top;
+      const uint2 e = stk[top * kBvhBlock];
+      n = (int)e.x;
+      down = key_beats(__int_as_float((int)e.y), best, s.box + (size_t)n * 6, p);
+    }
+    if (!down) break;
   }
   if (overflow) {
     atomicOr(status, 1);
@@ -424,21 +427,29 @@ void launch_metro_ep(const SurfaceDev& s, const double* ep, int nq, const double
 }
 
 
+// A walk is a chain of some 150 dependent steps for the longest of a wave's queries, and a wave
+// runs a leaf and an inner step in every round its lanes disagree. Few queries leave most of the
+// device idle whatever is done, so they are spread over more waves of fewer lanes: 488 queries on
+// 20,480 triangles take 257 us with 64 lanes, 234 with 32, 211 with 16, 191 with 8; 10,088
+// queries 248, 231, 272 and 284, and 411,080 queries 253, 321, 457 and 762.
+int closest_lanes(int nq) { return nq <= 2048 ? 8 : 64; }
+
 void launch_closest(const SurfaceDev& s, int nq, const double* P, int soa, int stride, const int* ids, double* S, int* I,
                     double* C, double* N, double* sqrD, int* status, hipStream_t st, const int* order) {
   if (nq <= 0) return;
-  const size_t lds = (size_t)stack_frames(s.depth) * kBvhBlock * sizeof(unsigned);
-  hipLaunchKernelGGL(closest_kernel, dim3((nq + kBvhBlock - 1) / kBvhBlock), dim3(kBvhBlock), lds, st, s,
-                     (const PatchSeg*)nullptr, 0, nq, P, soa, stride, ids, order, S, I, C, N, sqrD, status);
+  const size_t lds = (size_t)stack_frames(s.depth) * kBvhBlock * sizeof(uint2);
+  const int lanes = closest_lanes(nq), per_block = lanes * (kBvhBlock / 64);
+  hipLaunchKernelGGL(closest_kernel, dim3((nq + per_block - 1) / per_block), dim3(kBvhBlock), lds, st, s,
+                     (const PatchSeg*)nullptr, 0, lanes, nq, P, soa, stride, ids, order, S, I, C, N, sqrD, status);
 }
 
-void launch_closest_segs(const PatchSeg* segs, int nseg, int nblocks, int max_depth, const double* P, int soa,
+void launch_closest_segs(const PatchSeg* segs, int nseg, int nblocks, int lanes, int max_depth, const double* P, int soa,
                          int stride, const int* ids, const int* order, double* C, double* N, int* status,
                          hipStream_t st) {
   if (nseg <= 0 || nblocks <= 0) return;
-  const size_t lds = (size_t)stack_frames(max_depth) * kBvhBlock * sizeof(unsigned);
+  const size_t lds = (size_t)stack_frames(max_depth) * kBvhBlock * sizeof(uint2);
   SurfaceDev none{};
-  hipLaunchKernelGGL(closest_kernel, dim3(nblocks), dim3(kBvhBlock), lds, st, none, segs, nseg, 0, P, soa, stride,
+  hipLaunchKernelGGL(closest_kernel, dim3(nblocks), dim3(kBvhBlock), lds, st, none, segs, nseg, lanes, 0, P, soa, stride,
                      ids, order, (double*)nullptr, (int*)nullptr, C, N, (double*)nullptr, status);
 }
 

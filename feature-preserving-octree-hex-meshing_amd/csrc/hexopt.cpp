@@ -1308,6 +1308,7 @@ int hexopt_project_patches(hexopt_ctx* c, int npatch, hexopt_surface* const* pat
   // all patches in one launch: normal_T = pseudonormal N, dis_T = N . closest point
   std::vector<PatchSeg> segs;
   int nblocks = 0, max_depth = 1;
+  const int lanes = closest_lanes(nT), per_block = lanes * (kBvhBlock / 64);
   for (int p = 0; p < npatch; ++p) {
     const int n = c->patch_off[p + 1] - c->patch_off[p];
     if (n == 0) continue;
@@ -1317,7 +1318,7 @@ int hexopt_project_patches(hexopt_ctx* c, int npatch, hexopt_surface* const* pat
     g.q0 = c->patch_off[p];
     g.n = n;
     segs.push_back(g);
-    nblocks += (n + kBvhBlock - 1) / kBvhBlock;
+    nblocks += (n + per_block - 1) / per_block;
     max_depth = std::max(max_depth, patches[p]->view.depth);
   }
   if (segs.size() != c->h_segs.size() ||
@@ -1328,7 +1329,7 @@ int hexopt_project_patches(hexopt_ctx* c, int npatch, hexopt_surface* const* pat
     HIPCHK(c, hipMemcpyAsync(c->d_segs.p, c->h_segs.data(), segs.size() * sizeof(PatchSeg), hipMemcpyHostToDevice,
                              st));
   }
-  launch_closest_segs(c->d_segs.as<PatchSeg>(), (int)segs.size(), nblocks, max_depth, c->d_cur.as<double>(), 1,
+  launch_closest_segs(c->d_segs.as<PatchSeg>(), (int)segs.size(), nblocks, lanes, max_depth, c->d_cur.as<double>(), 1,
                       c->L.nV, c->d_tids.as<int>(), c->d_porder.as<int>(), c->d_pC.as<double>(),
                       const_cast<double*>(c->sd.t_n), c->d_pstat.as<int>(), st);
   launch_refold_planes(c->sd, c->d_trow.as<int>(), c->nrows, c->d_pC.as<double>(), const_cast<double*>(c->sd.t_d), c->d_S0.as<double>(),
