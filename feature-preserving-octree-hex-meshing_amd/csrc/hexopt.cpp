@@ -56,8 +56,8 @@ struct hexopt_ctx {
   MeshLayout L;
   std::string err;
   // layout on the device
-  DevBuf d_conn, d_tile_hex, d_tile_col, d_tile_lv, d_lv_gid, d_lv_slot, d_lv_first, d_lidx, d_tile_corner, d_sv_gid,
-      d_sv_off, d_sv_slots, d_lv_dst, d_v_dst;
+  DevBuf d_conn, d_tile_hex, d_tile_col, d_tile_lv, d_lv_gid, d_lv_slot, d_lidx, d_tile_corner, d_sv_gid,
+      d_sv_off, d_sv_slots, d_lv_pair, d_v_dst;
   DevBuf d_iso;  // vertices without hexes
   DevBuf d_vperm, d_rows;  // caller's id of every vertex; rows in the caller's order, in transit
   DevBuf d_torder;       // plane queries sorted by vertex (Morton) order
@@ -256,10 +256,9 @@ hexopt_ctx* hexopt_create(int nV, const double* V, int nH, const int32_t* hexes,
   rc |= upload(c, c->d_tile_lv, L.tile_lv);
   rc |= upload(c, c->d_lv_gid, L.lv_gid);
   rc |= upload(c, c->d_lv_slot, L.lv_slot);
-  rc |= upload(c, c->d_lv_first, L.lv_first);
   rc |= upload(c, c->d_lidx, L.lidx);
   rc |= upload(c, c->d_tile_corner, L.tile_corner);
-  rc |= upload(c, c->d_lv_dst, L.lv_dst);
+  rc |= upload(c, c->d_lv_pair, L.lv_pair);
   rc |= upload(c, c->d_v_dst, L.v_dst);
   rc |= upload(c, c->d_sv_gid, L.sv_gid);
   rc |= upload(c, c->d_sv_off, L.sv_off);
@@ -284,9 +283,9 @@ hexopt_ctx* hexopt_create(int nV, const double* V, int nH, const int32_t* hexes,
   }
   c->tm = TileMesh{L.nV, L.nH, L.nTiles, L.nShared, L.nSlots, c->d_conn.as<int>(), c->d_tile_hex.as<int>(),
                    c->d_tile_col.as<uint16_t>(), c->d_tile_lv.as<int>(), c->d_lv_gid.as<int>(),
-                   c->d_lv_slot.as<int>(), c->d_lv_first.as<uint8_t>(), c->d_lidx.as<uint16_t>(),
+                   c->d_lv_slot.as<int>(), c->d_lidx.as<uint16_t>(),
                    c->d_sv_gid.as<int>(), c->d_sv_off.as<int>(), c->d_sv_slots.as<int>(),
-                   c->d_tile_corner.as<uint8_t>(), c->d_lv_dst.as<int>(), c->d_v_dst.as<int>(),
+                   c->d_tile_corner.as<uint8_t>(), c->d_lv_pair.as<int>(), c->d_v_dst.as<int>(),
                    (int)L.lv_gid.size()};
   hexopt_constraints none{};
   if (hexopt_set_constraints(c, &none) != HEXOPT_OK) {

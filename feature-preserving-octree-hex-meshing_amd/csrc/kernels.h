@@ -15,13 +15,12 @@ struct TileMesh {
   const int* tile_lv;
   const int* lv_gid;
   const int* lv_slot;
-  const uint8_t* lv_first;
   const uint16_t* lidx;
   const int* sv_gid;
   const int* sv_off;
   const int* sv_slots;
   const uint8_t* tile_corner;
-  const int* lv_dst;  // per local vertex: place among all (tile, vertex) pairs, vertex by vertex
+  const int* lv_pair; // per local vertex: id (top bit: first tile) and place among all (tile, vertex) pairs
   const int* v_dst;   // nV+1: each vertex's run of places
   int nPairs;         // number of those pairs
 };
@@ -120,7 +119,7 @@ void launch_apply32_f64(const TileMesh& tm, const RefOp& ro, const float* K, con
 // updated x, r, z (zout may alias z); k is the CG iteration and last marks the final one (the
 // operator pass of cube references forms the previous iteration's beta step, so the one-block
 // beta pass runs only after the last update). Every tile writes E p of each of its vertices as a float4
-// at lv_dst (halo holds one float4 per (tile, vertex) pair); the update sums vertex v's run
+// at its place in lv_pair (halo holds one float4 per (tile, vertex) pair); the update sums vertex v's run
 // v_dst[v] .. v_dst[v+1]. iso lists the vertices without hexes.
 void launch_cg32_init(int nV, int nL, const SoftDev& sd, double prox, const float* b, const float* invd, float* x,
                       float* r, float* z, float* pprev, void* state, double* part_b, double* part_rz, double* part_q,

@@ -205,17 +205,27 @@ __device__ __forceinline__ void k_pair(const double* K, int nH, int h, int q, CT
   }
 }
 
+// the 8 local vertices of hex h, one 16-byte load
+__device__ __forceinline__ uint4 load_li(const TileMesh& tm, int h) { return reinterpret_cast<const uint4*>(tm.lidx)[h]; }
+__device__ __forceinline__ void unpack_li(const uint4& w, int li[8]) {
+  const unsigned v[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) { li[2 * k] = (int)(v[k] & 0xffffu); li[2 * k + 1] = (int)(v[k] >> 16); }
+}
+__device__ __forceinline__ void load_li(const TileMesh& tm, int h, int li[8]) { unpack_li(load_li(tm, h), li); }
+
 // Adds the tile's per-hex corner values c[8][NC] into its LDS accumulator (NC planes of
 // kMaxLV), without atomics and in a fixed order per vertex, so the sums are deterministic.
 // Tiles where no vertex sits at the same corner index of two hexes (tile_corner, true for
 // every tile of a consistently oriented grid) add corner k of all hexes in phase k: 8
 // phases with every thread busy. Other tiles add hex colour by colour. The caller has made
-// the accumulator's initial values visible (a barrier); the last phase ends in one.
+// the accumulator's initial values visible (a barrier); the last phase ends in one. corner is
+// tile_corner[tile], which the caller loads with the tile's ranges.
 template <class T, int NC>
-__device__ __forceinline__ void scatter_tile(const TileMesh& tm, int tile, int nh, bool active, const int li[8],
-                                             const T c[8][NC], T* acc) {
+__device__ __forceinline__ void scatter_tile(const TileMesh& tm, int tile, int corner, int nh, bool active,
+                                             const int li[8], const T c[8][NC], T* acc) {
   const int tid = threadIdx.x;
-  if (tm.tile_corner[tile]) {
+  if (corner) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (active) {
@@ -242,10 +252,10 @@ __device__ __forceinline__ void scatter_tile(const TileMesh& tm, int tile, int n
 
 // scatter_tile for 3 values per vertex kept as float4 in LDS (one 16-byte read-modify-write
 // per corner)
-__device__ __forceinline__ void scatter_tile4(const TileMesh& tm, int tile, int nh, bool active, const int li[8],
-                                              const float c[8][3], float4* acc) {
+__device__ __forceinline__ void scatter_tile4(const TileMesh& tm, int tile, int corner, int nh, bool active,
+                                              const int li[8], const float c[8][3], float4* acc) {
   const int tid = threadIdx.x;
-  if (tm.tile_corner[tile]) {
+  if (corner) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (active) {
@@ -304,11 +314,10 @@ void tile_scatter_kernel(TileMesh tm, Op op, T* halo, double* partial) {
     for (int j = 0; j < NC; ++j) c[k][j] = T(0);
   if (active) {
     op.hex(h0 + tid, c);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) li[k] = tm.lidx[(size_t)k * tm.nH + h0 + tid];
+    load_li(tm, h0 + tid, li);
   }
   __syncthreads();
-  scatter_tile<T, NC>(tm, tile, nh, active, li, c, acc);
+  scatter_tile<T, NC>(tm, tile, tm.tile_corner[tile], nh, active, li, c, acc);
   double part = 0.0;
   for (int lv = tid; lv < nlv; lv += kTileHex) {
     const int g = tm.lv_gid[lv0 + lv], s = tm.lv_slot[lv0 + lv];
@@ -1217,14 +1226,18 @@ __device__ void sum_parts_n(const double* const (&p)[N], int n, double* red, dou
 // (one round trip instead of U); the additions keep sum_parts_n's order, so the sums are the
 // same
 template <int N, int U>
-__device__ void sum_parts_n_wide(const double* const (&p)[N], int n, double* red, double out[N]) {
-  double v[U][N];
+__device__ __forceinline__ void load_parts_wide(const double* const (&p)[N], int n, double v[U][N]) {
 #pragma unroll
   for (int j = 0; j < U; ++j) {
     const int i = threadIdx.x + j * (int)blockDim.x;
 #pragma unroll
     for (int k = 0; k < N; ++k) v[j][k] = i < n ? p[k][i] : 0.0;
   }
+}
+
+template <int N, int U>
+__device__ __forceinline__ void add_parts_wide(const double* const (&p)[N], int n, const double v[U][N], double* red,
+                                               double out[N]) {
 #pragma unroll
   for (int k = 0; k < N; ++k) out[k] = 0;
 #pragma unroll
@@ -1239,6 +1252,13 @@ __device__ void sum_parts_n_wide(const double* const (&p)[N], int n, double* red
     for (int k = 0; k < N; ++k) out[k] += p[k][i];
   }
   block_sum_n<N>(out, red);
+}
+
+template <int N, int U>
+__device__ void sum_parts_n_wide(const double* const (&p)[N], int n, double* red, double out[N]) {
+  double v[U][N];
+  load_parts_wide<N, U>(p, n, v);
+  add_parts_wide<N, U>(p, n, v, red, out);
 }
 
 // Eigen ConjugateGradient.h:44-62 (zero rhs, early exit) and the first direction.
@@ -1492,8 +1512,7 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_kernel(TileMesh tm, RefOp
   int li[8];
   float kr[CUBE ? 48 : 1];
   if (active) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) li[k] = tm.lidx[(size_t)k * nH + h0 + tid];
+    load_li(tm, h0 + tid, li);
     if constexpr (CUBE) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) k_pair(K, nH, h0 + tid, q, kr + 12 * q);
@@ -1501,7 +1520,8 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_kernel(TileMesh tm, RefOp
   }
   // stage p of the tile's vertices
   for (int lv = tid; lv < nlv; lv += kTileHex) {
-    const int g = tm.lv_gid[lv0 + lv];
+    const int2 pair = reinterpret_cast<const int2*>(tm.lv_pair)[lv0 + lv];
+    const int g = pair.x & 0x7fffffff;
     float pv[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -1509,7 +1529,7 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_kernel(TileMesh tm, RefOp
       sp[d * kMaxLV + lv] = pv[d];
       acc[d * kMaxLV + lv] = 0.0f;
     }
-    if (tm.lv_first[lv0 + lv]) {
+    if (pair.x < 0) {
 #pragma unroll
       for (int d = 0; d < 3; ++d) pnew[(size_t)d * nV + g] = pv[d];
     }
@@ -1545,10 +1565,10 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_kernel(TileMesh tm, RefOp
       for (int d = 0; d < 3; ++d) e += q[k][d] * c[k][d];
     part = (double)e;
   }
-  scatter_tile<float, 3>(tm, tile, nh, active, li, c, acc);
+  scatter_tile<float, 3>(tm, tile, tm.tile_corner[tile], nh, active, li, c, acc);
   // E p of each local vertex to its place; the update sums each vertex's run
   for (int lv = tid; lv < nlv; lv += kTileHex)
-    halo[tm.lv_dst[lv0 + lv]] = make_float4(acc[lv], acc[kMaxLV + lv], acc[2 * kMaxLV + lv], 0.0f);
+    halo[tm.lv_pair[2 * (size_t)(lv0 + lv) + 1]] = make_float4(acc[lv], acc[kMaxLV + lv], acc[2 * kMaxLV + lv], 0.0f);
   const double bs = block_sum(part, red);
   if (tid == 0) partial[tile] = bs;
 }
@@ -1575,11 +1595,21 @@ __device__ __forceinline__ void line_row(const SoftDev& sd, int nV, const T* __r
 
 // The beta step of CG iteration up.k (cg32_beta_kernel's), formed by every block of the next
 // operator pass from the update pass's partials; block 0 records it in the state. Returns
-// whether the solve has converged (the pass then ends); red holds 5 * 16 values.
-__device__ __forceinline__ bool form_beta(CGState* st, const UpdParts& up, double* red, double& beta) {
+// whether the solve has ended (the pass then does too); done is the state's flag, loaded earlier so
+// that its latency overlaps the partials'; red holds 5 * 16 values.
+struct BetaParts {
+  double v[6][5];
+};
+__device__ __forceinline__ void load_beta(const UpdParts& up, BetaParts& b) {
+  const double* const parts[5] = {up.p[0], up.p[1], up.p[2], up.p[3], up.p[4]};
+  load_parts_wide<5, 6>(parts, up.n, b.v);
+}
+__device__ __forceinline__ bool form_beta(CGState* st, const UpdParts& up, const BetaParts& b, int done, double* red,
+                                          double& beta) {
   const double* const parts[5] = {up.p[0], up.p[1], up.p[2], up.p[3], up.p[4]};
   double v[5];
-  sum_parts_n_wide<5, 6>(parts, up.n, red, v);
+  add_parts_wide<5, 6>(parts, up.n, b.v, red, v);
+  if (done) return true;  // ended before: the partials are an earlier step's
   const double rr = v[0], rz = v[1];
   const bool conv = rr < st->threshold;
   const double absOld = st->hist[up.k & 1];
@@ -1607,9 +1637,8 @@ __device__ __forceinline__ bool form_beta(CGState* st, const UpdParts& up, doubl
 // of its E p, first-writer flag; at most kMaxLV / kTileHex = 4 per thread), its hex's corner
 // ids and 48 operator values.
 struct PipeTile {
-  int h0, nh, lv0, nlv;
-  int g[kMaxLV / kTileHex], s[kMaxLV / kTileHex];
-  unsigned first;  // bit j: local vertex tid + j * kTileHex writes p
+  int h0, nh, lv0, nlv, corner;
+  int2 v[kMaxLV / kTileHex];  // id (top bit: this tile writes p) and place of E p
   int li[8];
   float kr[48];
 };
@@ -1620,21 +1649,37 @@ __device__ __forceinline__ void pipe_fetch(const TileMesh& tm, const float* __re
   P.nh = tm.tile_hex[t + 1] - P.h0;
   P.lv0 = tm.tile_lv[t];
   P.nlv = tm.tile_lv[t + 1] - P.lv0;
-  P.first = 0;
+  P.corner = tm.tile_corner[t];
 #pragma unroll
   for (int j = 0; j < kMaxLV / kTileHex; ++j) {
     const int lv = tid + j * kTileHex;
-    if (lv < P.nlv) {
-      P.g[j] = tm.lv_gid[P.lv0 + lv];
-      P.s[j] = tm.lv_dst[P.lv0 + lv];
-      P.first |= tm.lv_first[P.lv0 + lv] ? (1u << j) : 0u;
-    }
+    if (lv < P.nlv) P.v[j] = reinterpret_cast<const int2*>(tm.lv_pair)[P.lv0 + lv];
   }
   if (tid < P.nh) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) P.li[k] = tm.lidx[(size_t)k * tm.nH + P.h0 + tid];
+    load_li(tm, P.h0 + tid, P.li);
 #pragma unroll
     for (int q = 0; q < 4; ++q) k_pair(K, tm.nH, P.h0 + tid, q, P.kr + 12 * q);
+  }
+}
+
+// z and the previous direction at a tile's local vertices (this thread's share), to be combined
+// once beta is known; fetched while the tile before is stored (the pass on 1.1M hexes 92.6 -> 87.9
+// us, on 262,144 27.3 -> 25.0). A compact tile of 256 hexes has about 400 of them, so two rounds of the
+// block are fetched ahead; what a ragged tile has beyond them is loaded where it is staged.
+constexpr int kAhead = 2;
+template <class T, class TILE>
+__device__ __forceinline__ void pipe_gather(const TILE& P, int nV, const T* __restrict__ z,
+                                            const T* __restrict__ pprev, bool prev, T zr[kAhead][3], T pr[kAhead][3]) {
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j) {
+    if ((int)threadIdx.x + j * kTileHex < P.nlv) {
+      const int g = P.v[j].x & 0x7fffffff;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        zr[j][d] = z[(size_t)d * nV + g];
+        pr[j][d] = prev ? pprev[(size_t)d * nV + g] : T(0);
+      }
+    }
   }
 }
 
@@ -1652,7 +1697,7 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_pipe_kernel(TileMesh tm, 
   __shared__ float4 sp[kMaxLV];
   __shared__ float4 acc[kMaxLV];
   __shared__ double red[5 * 16];
-  if (st->done) return;
+  const int done = st->done;
   const int tid = threadIdx.x;
   const int nV = tm.nV, nT = tm.nTiles;
   const int q8 = nT / 8, r8 = nT % 8;
@@ -1660,15 +1705,22 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_pipe_kernel(TileMesh tm, 
   const int nb = ((int)gridDim.x + 7 - x) / 8;  // blocks on XCD x
   const int tend = (x + 1) * q8 + (x + 1 < r8 ? x + 1 : r8);
   int tile = x * q8 + (x < r8 ? x : r8) + rank;
+  BetaParts bp;
+  if (up.n > 0) load_beta(up, bp);
   PipeTile P;
-  if (tile < tend) pipe_fetch(tm, K, tile, P);
+  float zr[kAhead][3], pr[kAhead][3];
+  if (tile < tend) {
+    pipe_fetch(tm, K, tile, P);
+    pipe_gather(P, nV, z, pprev, true, zr, pr);
+  }
   // (the first tile's loads are in flight while the beta step is formed)
   float beta;
   if (up.n > 0) {
     double bt;
-    if (form_beta(st, up, red, bt)) return;
+    if (form_beta(st, up, bp, done, red, bt)) return;
     beta = (float)bt;
   } else {
+    if (done) return;
     beta = (float)st->beta;
   }
   // the work outside the tiles, spread over all blocks: line unknowns, and p of the
@@ -1687,13 +1739,15 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_pipe_kernel(TileMesh tm, 
     for (int j = 0; j < kMaxLV / kTileHex; ++j) {
       const int lv = tid + j * kTileHex;
       if (lv < P.nlv) {
-        const int g = P.g[j];
+        const int g = P.v[j].x & 0x7fffffff;
         float pv[3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) pv[d] = z[(size_t)d * nV + g] + beta * pprev[(size_t)d * nV + g];
+        for (int d = 0; d < 3; ++d)
+          pv[d] = j < kAhead ? zr[j % kAhead][d] + beta * pr[j % kAhead][d]
+                             : z[(size_t)d * nV + g] + beta * pprev[(size_t)d * nV + g];
         sp[lv] = make_float4(pv[0], pv[1], pv[2], 0.0f);
         acc[lv] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (P.first & (1u << j)) {
+        if (P.v[j].x < 0) {
 #pragma unroll
           for (int d = 0; d < 3; ++d) pnew[(size_t)d * nV + g] = pv[d];
         }
@@ -1727,15 +1781,15 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_pipe_kernel(TileMesh tm, 
       part += (double)e;
     }
     // this tile's indices, then the next tile's loads
-    const int cur = tile, nh = P.nh, nlv = P.nlv;
-    int li[8], g[kMaxLV / kTileHex], sl[kMaxLV / kTileHex];
+    const int cur = tile, nh = P.nh, nlv = P.nlv, corner = P.corner;
+    int li[8], sl[kMaxLV / kTileHex];
 #pragma unroll
     for (int k = 0; k < 8; ++k) li[k] = P.li[k];
 #pragma unroll
-    for (int j = 0; j < kMaxLV / kTileHex; ++j) { g[j] = P.g[j]; sl[j] = P.s[j]; }
+    for (int j = 0; j < kMaxLV / kTileHex; ++j) sl[j] = P.v[j].y;
     tile += nb;
     if (tile < tend) pipe_fetch(tm, K, tile, P);
-    scatter_tile4(tm, cur, nh, active, li, c, acc);
+    scatter_tile4(tm, cur, corner, nh, active, li, c, acc);
 #pragma unroll
     for (int j = 0; j < kMaxLV / kTileHex; ++j) {
       const int lv = tid + j * kTileHex;
@@ -1743,6 +1797,7 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_pipe_kernel(TileMesh tm, 
         halo[sl[j]] = acc[lv];
       }
     }
+    if (tile < tend) pipe_gather(P, nV, z, pprev, true, zr, pr);
     // the next tile's staging overwrites sp and acc
     __syncthreads();
   }
@@ -1803,27 +1858,18 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
                                                         double* part_rr, double* part_rz, double* part_qz,
                                                         double* part_bzq, double* part_qq) {
   __shared__ double red[5 * 16];
-  if (st->done) return;
+  const int done = st->done;
   const int nV = tm.nV;
   const size_t nA = 3 * (size_t)nV;
-  T alpha;
-  if (ntiles > 0) {
-    const double* const pt[1] = {part_tile};
-    double ev[1];
-    sum_parts_n_wide<1, 4>(pt, ntiles, red, ev);
-    const double e = ev[0];
-    const double b = (double)(T)st->beta;
-    alpha = (T)(st->absNew / (e + st->qz + 2.0 * b * st->bzq + b * b * st->qq));
-  } else {
-    alpha = (T)st->alpha;
-  }
-  double srr = 0, srz = 0, fz = 0, fzq = 0, fq = 0;
-  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < nV; g += gridDim.x * blockDim.x) {
-    // every load that does not wait on another goes out first: the vertex's run bounds, its
-    // p, r, x, 1/diag and constraint row; then the R rows (which wait only on the constraint
-    // row) and the run of E p places (one per tile holding the vertex, in tile order)
-    const int k0 = tm.v_dst[g], k1 = tm.v_dst[g + 1];
-    T pf[3], rf[3], xf[3], df[3];
+  // every load of a vertex that does not wait on another goes out together: its run bounds, its
+  // p, r, x, 1/diag and constraint row. The first vertex's go out before alpha is formed, whose
+  // partials take as long to come
+  int k0, k1;
+  T pf[3], rf[3], xf[3], df[3];
+  int2 cl;
+  auto load = [&](int g) {
+    k0 = tm.v_dst[g];
+    k1 = tm.v_dst[g + 1];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       const size_t j = (size_t)d * nV + g;
@@ -1832,7 +1878,28 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
       xf[d] = x[j];
       df[d] = invd[j];
     }
-    const int2 cl = sd.cl ? reinterpret_cast<const int2*>(sd.cl)[g] : make_int2(-1, -1);
+    cl = sd.cl ? reinterpret_cast<const int2*>(sd.cl)[g] : make_int2(-1, -1);
+  };
+  int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < nV) load(g);
+  T alpha;
+  if (ntiles > 0) {
+    const double* const pt[1] = {part_tile};
+    double ev[1];
+    sum_parts_n_wide<1, 4>(pt, ntiles, red, ev);
+    if (done) return;
+    const double e = ev[0];
+    const double b = (double)(T)st->beta;
+    alpha = (T)(st->absNew / (e + st->qz + 2.0 * b * st->bzq + b * b * st->qq));
+  } else {
+    if (done) return;
+    alpha = (T)st->alpha;
+  }
+  double srr = 0, srz = 0, fz = 0, fzq = 0, fq = 0;
+  for (bool first = true; g < nV; g += gridDim.x * blockDim.x, first = false) {
+    if (!first) load(g);
+    // then the R rows (which wait only on the constraint row) and the run of E p places (one per
+    // tile holding the vertex, in tile order)
     const int ci = cl.x, ln = cl.y;
     double pv[3];
 #pragma unroll
@@ -1892,33 +1959,74 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
 // now 165 us for the operator pass and 78 us for the vector pass.
 
 // The operator pass. Persistent blocks, the tiles of an XCD dealt as in cg32_apply_pipe_kernel.
-// A hex's 48 FP64 operator values alone would fill 96 registers, so nothing is fetched a tile
+// A hex's 48 FP64 operator values alone would fill 96 registers, so nothing is held for a tile
 // ahead: the corner values stay in LDS and are read again by every tet, the operator values come
 // pair by pair, and the registers this leaves free let three blocks share a CU and cover each
-// other's loads. start: the pass that forms E x for the first residual (z = the positions, no
-// direction before it, a_L = 0).
-template <bool CUBE>
+// other's loads. (With the next tile's ids, z and p fetched ahead, 30 to 90 registers spill.)
+// What a block waits for before its first tile is a chain of loads, and on a mesh of a few tiles
+// that chain is the pass: so the first tile's z and previous direction go to LDS, where they need
+// no registers, while the partials of beta are on their way, and are combined once beta is known.
+// Per call, loads after beta and as here: 150 -> 144 us on 1.1M hexes, 35.4 -> 33.3 us on 262,144,
+// 8.8 -> 7.7 us on 729.
+// START: the pass that forms E x for the first residual (z = the positions, no direction before
+// it, a_L = 0).
+template <bool CUBE, bool START>
 __global__ __launch_bounds__(kTileHex, CUBE ? 3 : 2) void cg64_apply_kernel(TileMesh tm, RefOp ro, const double* __restrict__ K,
                                                                  const double* __restrict__ z,
                                                                  const double* __restrict__ pprev,
                                                                  double* __restrict__ pnew, double* __restrict__ out,
                                                                  double* __restrict__ halo, SoftDev sd,
                                                                  const int* __restrict__ iso, int niso, CGState* st,
-                                                                 double* partial, UpdParts up, int start) {
+                                                                 double* partial, UpdParts up) {
   __shared__ double sp[3 * kMaxLV];
   __shared__ double acc[3 * kMaxLV];
   __shared__ double red[5 * 16];
-  double beta = 0.0;
-  if (!start) {
-    if (st->done) return;
-    if (up.n > 0 && form_beta(st, up, red, beta)) return;
-  }
   const int tid = threadIdx.x;
   const int nV = tm.nV, nH = tm.nH, nT = tm.nTiles;
   const size_t nA = 3 * (size_t)nV;
+  const int q8 = nT / 8, r8 = nT % 8;
+  const int x = blockIdx.x % 8, rank = blockIdx.x / 8;
+  const int nb = ((int)gridDim.x + 7 - x) / 8;  // blocks on XCD x
+  const int tend = (x + 1) * q8 + (x + 1 < r8 ? x + 1 : r8);
+  int tile = x * q8 + (x < r8 ? x : r8) + rank;
+  int h0 = 0, nh = 0, lv0 = 0, nlv = 0, corner = 0;
+  auto head = [&]() {
+    h0 = tm.tile_hex[tile];
+    nh = tm.tile_hex[tile + 1] - h0;
+    lv0 = tm.tile_lv[tile];
+    nlv = tm.tile_lv[tile + 1] - lv0;
+    corner = tm.tile_corner[tile];
+  };
+  double beta = 0.0;
+  bool raw = false;  // the tile's z is in sp and its previous direction in acc
+  if constexpr (START) {
+    if (tile < tend) head();
+  } else {
+    const int done = st->done;
+    BetaParts bp;
+    if (up.n > 0) load_beta(up, bp);
+    if (tile < tend) {
+      head();
+      for (int lv = tid; lv < nlv; lv += kTileHex) {
+        const int g = tm.lv_pair[2 * (size_t)(lv0 + lv)] & 0x7fffffff;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const size_t j = (size_t)d * nV + g;
+          sp[d * kMaxLV + lv] = z[j];
+          acc[d * kMaxLV + lv] = pprev[j];
+        }
+      }
+      raw = true;
+    }
+    if (up.n > 0) {
+      if (form_beta(st, up, bp, done, red, beta)) return;
+    } else if (done) {
+      return;
+    }
+  }
   // the work outside the tiles: line unknowns, and p of the vertices without hexes
   for (int i = blockIdx.x * kTileHex + tid; i < sd.nL; i += gridDim.x * kTileHex) {
-    if (start) {
+    if constexpr (START) {
       const int v = sd.lv[i];
       const double* t = sd.lt + (size_t)i * 3;
       double tp = 0;
@@ -1935,35 +2043,27 @@ __global__ __launch_bounds__(kTileHex, CUBE ? 3 : 2) void cg64_apply_kernel(Tile
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       const size_t j = (size_t)d * nV + g;
-      pnew[j] = start ? z[j] : z[j] + beta * pprev[j];
+      pnew[j] = START ? z[j] : z[j] + beta * pprev[j];
     }
   }
-  const int q8 = nT / 8, r8 = nT % 8;
-  const int x = blockIdx.x % 8, rank = blockIdx.x / 8;
-  const int nb = ((int)gridDim.x + 7 - x) / 8;  // blocks on XCD x
-  const int tend = (x + 1) * q8 + (x + 1 < r8 ? x + 1 : r8);
   double part = 0.0;
-  for (int tile = x * q8 + (x < r8 ? x : r8) + rank; tile < tend; tile += nb) {
-    const int h0 = tm.tile_hex[tile], nh = tm.tile_hex[tile + 1] - h0;
-    const int lv0 = tm.tile_lv[tile], nlv = tm.tile_lv[tile + 1] - lv0;
+  while (tile < tend) {
     const bool active = tid < nh;
     int li[8];
     double kp[2][12];
     if (active) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) li[k] = tm.lidx[(size_t)k * nH + h0 + tid];
+      load_li(tm, h0 + tid, li);
       if constexpr (CUBE) k_pair(K, nH, h0 + tid, 0, kp[0]);
     }
     for (int lv = tid; lv < nlv; lv += kTileHex) {
-      const int g = tm.lv_gid[lv0 + lv];
-      const bool first = tm.lv_first[lv0 + lv] != 0;
+      const int2 pair = reinterpret_cast<const int2*>(tm.lv_pair)[lv0 + lv];
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const size_t j = (size_t)d * nV + g;
-        const double pv = start ? z[j] : z[j] + beta * pprev[j];
+        const size_t j = (size_t)d * nV + (pair.x & 0x7fffffff);
+        const double pv = START ? z[j] : raw ? sp[d * kMaxLV + lv] + beta * acc[d * kMaxLV + lv] : z[j] + beta * pprev[j];
         sp[d * kMaxLV + lv] = pv;
         acc[d * kMaxLV + lv] = 0.0;
-        if (first) pnew[j] = pv;
+        if (pair.x < 0) pnew[j] = pv;
       }
     }
     __syncthreads();
@@ -2014,12 +2114,15 @@ __global__ __launch_bounds__(kTileHex, CUBE ? 3 : 2) void cg64_apply_kernel(Tile
           for (int d = 0; d < 3; ++d) part += sp[d * kMaxLV + li[k]] * c[k][d];
       }
     }
-    scatter_tile<double, 3>(tm, tile, nh, active, li, c, acc);
+    scatter_tile<double, 3>(tm, tile, corner, nh, active, li, c, acc);
     for (int lv = tid; lv < nlv; lv += kTileHex) {
-      const int k = tm.lv_dst[lv0 + lv];
+      const int k = tm.lv_pair[2 * (size_t)(lv0 + lv) + 1];
 #pragma unroll
       for (int d = 0; d < 3; ++d) halo[(size_t)d * tm.nPairs + k] = acc[d * kMaxLV + lv];
     }
+    tile += nb;
+    if (tile < tend) head();
+    raw = false;
     __syncthreads();  // the next tile's staging overwrites sp and acc
   }
   const double bs = block_sum(part, red);
@@ -3008,7 +3111,7 @@ int apply64_grid(int ntiles) {
   if (dev < 0 || dev >= 64) return std::min(ntiles, 8);
   if (fit[dev] == 0) {
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cg64_apply_kernel<CUBE>, kTileHex, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cg64_apply_kernel<CUBE, false>, kTileHex, 0) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       per_cu = cus = 0;
     fit[dev] = std::max(8, per_cu * cus);
@@ -3021,12 +3124,10 @@ int cg64_apply(const TileMesh& tm, const RefOp& ro, const double* K, const SoftD
                hipStream_t st) {
   const bool cube = ro.mode == REF_CUBE;
   const int grid = std::max(1, cube ? apply64_grid<true>(tm.nTiles) : apply64_grid<false>(tm.nTiles));
-  if (cube)
-    hipLaunchKernelGGL(cg64_apply_kernel<true>, dim3(grid), dim3(kTileHex), 0, st, tm, ro, K, z, pprev, pnew, w.out,
-                       w.halo, sd, iso, niso, (CGState*)w.state, w.part[2], up, start);
-  else
-    hipLaunchKernelGGL(cg64_apply_kernel<false>, dim3(grid), dim3(kTileHex), 0, st, tm, ro, K, z, pprev, pnew, w.out,
-                       w.halo, sd, iso, niso, (CGState*)w.state, w.part[2], up, start);
+  const auto kernel = cube ? (start ? cg64_apply_kernel<true, true> : cg64_apply_kernel<true, false>)
+                              : (start ? cg64_apply_kernel<false, true> : cg64_apply_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kTileHex), 0, st, tm, ro, K, z, pprev, pnew, w.out, w.halo, sd, iso, niso,
+                     (CGState*)w.state, w.part[2], up);
   return grid;
 }
 }  // namespace

@@ -189,13 +189,13 @@ bool build_layout(int nV, const double* V, int nH, const int* H, MeshLayout& L, 
     std::sort(lv.begin(), lv.end());
     for (size_t j = 0; j < lv.size(); ++j) local[lv[j]] = (int)j;
     for (int i = L.tile_hex[t]; i < L.tile_hex[t + 1]; ++i)
-      for (int k = 0; k < 8; ++k) L.lidx[(size_t)k * nH + i] = (uint16_t)local[L.conn[(size_t)k * nH + i]];
+      for (int k = 0; k < 8; ++k) L.lidx[(size_t)i * 8 + k] = (uint16_t)local[L.conn[(size_t)k * nH + i]];
     {
       std::vector<uint8_t> seen(lv.size(), 0);
       uint8_t ok = 1;
       for (int i = L.tile_hex[t]; i < L.tile_hex[t + 1]; ++i)
         for (int k = 0; k < 8; ++k) {
-          uint8_t& m = seen[L.lidx[(size_t)k * nH + i]];
+          uint8_t& m = seen[L.lidx[(size_t)i * 8 + k]];
           if (m & (1u << k)) ok = 0;
           m |= (uint8_t)(1u << k);
         }
@@ -203,17 +203,17 @@ bool build_layout(int nV, const double* V, int nH, const int* H, MeshLayout& L, 
     }
     for (int v : lv) {
       L.lv_gid.push_back(v);
-      L.lv_dst.push_back(L.v_dst[v] + dst_count[v]++);
+      const bool first = dst_count[v] == 0;
+      L.lv_pair.push_back(first ? v | (int)0x80000000u : v);
+      L.lv_pair.push_back(L.v_dst[v] + dst_count[v]++);
       if (ntiles_of_v[v] > 1) {
         // slots are numbered vertex by vertex (each vertex's in tile order), so the fold of a
         // vertex reads one contiguous run
         const int s = vslot_start[v] + slot_count[v];
         L.lv_slot.push_back(s);
-        L.lv_first.push_back(slot_count[v] == 0 ? 1 : 0);
         L.sv_slots[vslot_start[v] + slot_count[v]++] = s;
       } else {
         L.lv_slot.push_back(-1);
-        L.lv_first.push_back(1);
       }
       local[v] = -1;
     }

@@ -29,11 +29,12 @@ struct MeshLayout {
   std::vector<int> tile_lv;     // nTiles+1 local-vertex ranges
   std::vector<int> lv_gid;      // local vertex -> new vertex id
   std::vector<int> lv_slot;     // -1: written directly; else halo slot
-  std::vector<uint8_t> lv_first;  // 1: the vertex is this tile's alone, or this tile holds its
-                                  //    first halo slot (the one tile that writes per-vertex data)
-  std::vector<uint16_t> lidx;   // [8][nH] local vertex of each corner within its tile
-  std::vector<int> lv_dst;      // per local vertex: its place among all (tile, vertex) pairs,
-                                // numbered vertex by vertex (each vertex's in tile order)
+  std::vector<uint16_t> lidx;   // [nH][8] local vertex of each corner within its tile
+  std::vector<int> lv_pair;     // per local vertex two ints, read together: its new vertex id,
+                                // with the top bit set in the first tile that holds it (the one
+                                // that writes per-vertex data), and its place among all (tile,
+                                // vertex) pairs, numbered vertex by vertex (each vertex's in tile
+                                // order)
   std::vector<int> v_dst;       // nV+1: vertex v's run of places in that numbering
   std::vector<uint8_t> tile_corner;  // 1: no vertex of the tile sits at the same corner index of
                                      // two of its hexes, so corner k of every hex can be added in
