@@ -1510,8 +1510,8 @@ void hexopt_octree_destroy(hexopt_octree* o) { delete o; }
 
 int hexopt_octree_sizes(const hexopt_octree* o, int64_t* out4, double* ms) {
   if (!o || !out4) return HEXOPT_EINVAL;
-  out4[0] = (int64_t)(o->r.leaves.size() / 4);
-  out4[1] = (int64_t)(o->r.nodes.size() / 3);
+  out4[0] = o->r.leaves;
+  out4[1] = o->r.nodes;
   out4[2] = o->r.levels;
   out4[3] = o->r.evaluated;
   if (ms) *ms = o->r.ms;
@@ -1520,11 +1520,12 @@ int hexopt_octree_sizes(const hexopt_octree* o, int64_t* out4, double* ms) {
 
 int hexopt_octree_copy(const hexopt_octree* o, int32_t* leaves, int32_t* nodes, double* V, int32_t* H) {
   if (!o) return HEXOPT_EINVAL;
-  if (leaves) std::copy(o->r.leaves.begin(), o->r.leaves.end(), leaves);
-  if (nodes) std::copy(o->r.nodes.begin(), o->r.nodes.end(), nodes);
-  if (V) std::copy(o->r.V.begin(), o->r.V.end(), V);
-  if (H) std::copy(o->r.hexes.begin(), o->r.hexes.end(), H);
-  return HEXOPT_OK;
+  g_octree_error.clear();
+  const OnDevice on(o->device);
+  std::string err;
+  if (octree_copy(*o->dev, o->r, leaves, nodes, V, H, err)) return HEXOPT_OK;
+  g_octree_error = err;
+  return HEXOPT_EHIP;
 }
 
 struct hexopt_curves {

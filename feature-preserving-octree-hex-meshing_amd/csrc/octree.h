@@ -12,13 +12,11 @@
 namespace hexopt {
 
 struct OctreeOut {
-  std::vector<int32_t> leaves;  // n x 4: x, y, z, extent (voxel units), level by level
-  std::vector<int32_t> nodes;   // m x 3: integer node positions
-  std::vector<double> V;        // m x 3: base + voxel_size * node position
-  std::vector<int32_t> hexes;   // n x 8: node ids of each leaf's corners, reference corner order
-  int levels = 0;               // number of levels holding leaves (deepest leaf level + 1)
-  long evaluated = 0;           // predicate evaluations
-  double ms = 0;                // device time of the subdivision (hipEvents on its stream)
+  int64_t leaves = 0;  // rows of each of the results, which stay on the device (octree_copy)
+  int64_t nodes = 0;
+  int levels = 0;      // number of levels holding leaves (deepest leaf level + 1)
+  long evaluated = 0;  // predicate evaluations
+  double ms = 0;       // device time of the subdivision (hipEvents on its stream)
 };
 
 // Device state of one octree: a dense byte grid of split flags per level. grid: cells per axis
@@ -33,10 +31,16 @@ void octree_destroy(OctreeDev* o);
 // OctreeGrid::subdivide(predicate, graded, paired) of a fresh octree (octree.cpp:648-690: its
 // queue starts from the root cells) when cells is null; the targeted variant over n listed cells (x, y, z, extent rows, host
 // memory; octree.cpp:691-729: a listed cell that is a leaf and passes the predicate is split,
-// its children are not tested) otherwise. Then the leaves, nodes and hexes of the result into
-// out (ms: device time of the subdivision). False with a message on a bad grid or cell, a
+// its children are not tested) otherwise. Then the leaves, nodes and hexes of the result, on the
+// device; their sizes go into out (ms: device time of the subdivision). False with a message on a bad grid or cell, a
 // level above 2^31 cells or a device error.
 bool octree_timed(OctreeDev& o, const SurfaceDev* s, int stop_extent, int n, const int* cells, hipStream_t st,
                   OctreeOut& out, std::string& err);
+// The results of the last octree_timed into host memory, each that is not null: leaves n x 4
+// (x, y, z, extent in voxel units, level by level), nodes m x 3 (integer positions), V m x 3
+// (base + voxel_size * position), hexes n x 8 (node ids of each leaf's corners, reference corner
+// order). The device they were built on has to be current.
+bool octree_copy(const OctreeDev& o, const OctreeOut& out, int32_t* leaves, int32_t* nodes, double* V,
+                 int32_t* hexes, std::string& err);
 
 }  // namespace hexopt

@@ -517,8 +517,10 @@ class Octree:
         nodes = np.empty((m, 3), np.int32)
         V = np.empty((m, 3), np.float64)
         H = np.empty((n, 8), np.int32)
-        lib().hexopt_octree_copy(C.c_void_p(self.h), leaves.ctypes.data, nodes.ctypes.data, V.ctypes.data,
-                                 H.ctypes.data)
+        rc = lib().hexopt_octree_copy(C.c_void_p(self.h), leaves.ctypes.data, nodes.ctypes.data, V.ctypes.data,
+                                      H.ctypes.data)
+        if rc:
+            raise RuntimeError("hexopt_octree_copy (%d): %s" % (rc, lib().hexopt_octree_error().decode()))
         return dict(leaves=leaves, nodes=nodes, V=V, H=H, levels=int(sz[2]), evaluated=int(sz[3]), ms=ms.value)
 
     def close(self):

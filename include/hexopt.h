@@ -304,7 +304,8 @@ int hexopt_octree_refine(hexopt_octree* o, hexopt_surface* s, int stop_extent, i
 /* leaves[n][4] (x, y, z, extent), nodes[m][3] (integer positions), V[m][3]
  * (mesh_transform + origin + voxel_size * position, octree_mesh's mo.V) and H[n][8] (node
  * ids of each leaf's corners in the reference's corner order, octree_mesh's mo.Hs); any may
- * be NULL. */
+ * be NULL. The results stay on the octree's device until it is destroyed or refined and are
+ * copied from there: HEXOPT_EHIP if the device fails (hexopt_octree_error() says why). */
 int hexopt_octree_copy(const hexopt_octree* o, int32_t* leaves, int32_t* nodes, double* V, int32_t* H);
 
 /* ---- feature-curve projection (LINE branch of dirty_graph_projection,
