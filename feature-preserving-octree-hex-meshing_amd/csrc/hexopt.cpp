@@ -61,16 +61,19 @@ struct hexopt_ctx {
   DevBuf d_iso;  // vertices without hexes
   DevBuf d_vperm, d_rows;  // caller's id of every vertex; rows in the caller's order, in transit
   DevBuf d_torder;       // plane queries sorted by vertex (Morton) order
-  DevBuf d_cgsave;       // CG state of the last direction solve, read back with the line search
   int n_iso = 0;
   TileMesh tm{};
   // positions (SoA, Morton numbering)
   DevBuf d_rest, d_cur;
   // reference operator
-  DevBuf d_invs, d_B, d_hflag, d_count;
+  DevBuf d_invs, d_B, d_hflag;
   int ref_mode = -1;
   // SLIM state
-  DevBuf d_K, d_rhs, d_invd, d_x, d_r, d_z, d_p, d_p2, d_tmp, d_halo, d_cg, d_part[8], d_scal;
+  DevBuf d_K, d_rhs, d_invd, d_x, d_r, d_z, d_p, d_p2, d_tmp, d_halo, d_part[8];
+  // what the host reads back, in one device block and one pinned copy of it, so that a line search
+  // takes one transfer: 16 scalars, the CG state, the state of the last direction solve, counters
+  DevBuf d_scal;
+  char* h_read = nullptr;
   // constraints
   DevBuf d_cidx, d_cl, d_S, d_b, d_cline, d_bids, d_bpos, d_cids, d_cpos, d_tids, d_tn, d_td, d_lv, d_lt, d_lo, d_rhs_a,
       d_invd_a, d_aL;
@@ -98,7 +101,7 @@ struct hexopt_ctx {
   DevBuf d_porder, d_pC, d_pstat, d_segs;
   bool lines_refreshable = false;
   // FP32 optimiser state
-  DevBuf f_K, f_rhs, f_invd, f_d, f_r, f_z, f_p, f_p2, f_tmp, f_e, f_halo, d_Ld64, d_halo64b, d_ninv, d_b64;
+  DevBuf f_K, f_rhs, f_invd, f_d, f_r, f_z, f_p, f_p2, f_tmp, f_e, f_halo, d_Ld64, d_halo64b, d_b64;
 };
 
 namespace {
@@ -163,6 +166,34 @@ int nblocks(long n) { long b = (n + 255) / 256; if (b < 1) b = 1; if (b > 2048) 
 
 RefOp refop(hexopt_ctx* c) { return RefOp{c->ref_mode, c->d_invs.as<double>(), c->d_B.as<double>()}; }
 
+// the parts of the block the host reads back
+size_t cg_bytes() { return (cg_state_bytes() + 15) / 16 * 16; }
+size_t read_bytes() { return 16 * sizeof(double) + 2 * cg_bytes() + 16; }
+void* cg_state(hexopt_ctx* c) { return c->d_scal.as<char>() + 16 * sizeof(double); }
+void* cg_saved(hexopt_ctx* c) { return c->d_scal.as<char>() + 16 * sizeof(double) + cg_bytes(); }
+int* counter(hexopt_ctx* c) { return (int*)(c->d_scal.as<char>() + 16 * sizeof(double) + 2 * cg_bytes()); }
+int ensure_read(hexopt_ctx* c) {
+  HIPCHK(c, c->d_scal.ensure(read_bytes()));
+  if (!c->h_read) HIPCHK(c, hipHostMalloc((void**)&c->h_read, read_bytes()));
+  return HEXOPT_OK;
+}
+// the block as it is when the stream has done all that is queued
+struct ReadBack {
+  const double* scal;
+  const void *cg, *saved;
+  int count;
+};
+int read_back(hexopt_ctx* c, ReadBack& r) {
+  HIPCHK(c, hipMemcpyAsync(c->h_read, c->d_scal.p, read_bytes(), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  r.scal = (const double*)c->h_read;
+  r.cg = c->h_read + 16 * sizeof(double);
+  r.saved = c->h_read + 16 * sizeof(double) + cg_bytes();
+  r.count = *(const int*)(c->h_read + 16 * sizeof(double) + 2 * cg_bytes());
+  return HEXOPT_OK;
+}
+
 // Scratch sized for the current mesh and constraints.
 int ensure_state(hexopt_ctx* c) {
   const int nV = c->L.nV, nH = c->L.nH;
@@ -173,12 +204,11 @@ int ensure_state(hexopt_ctx* c) {
   // 6 values per halo slot in the local step, 3 per (tile, vertex) pair in the CG
   HIPCHK(c, c->d_halo.ensure(std::max((size_t)6 * (c->L.nSlots + 1), (size_t)3 * (c->L.lv_gid.size() + 1)) *
                              sizeof(double)));
-  HIPCHK(c, c->d_cg.ensure(cg_state_bytes()));
   const size_t np = (size_t)std::max(std::max(std::max(c->L.nTiles, nblocks(n)), (nH + 255) / 256 + 1),
                                      std::max(2048, (nV + c->nL + 255) / 256 + 1)) + 64;
   const size_t npf = (size_t)(c->L.nShared + 255) / 256 + 1;
   for (int i = 0; i < 8; ++i) HIPCHK(c, c->d_part[i].ensure(std::max(np, npf) * sizeof(double)));
-  HIPCHK(c, c->d_scal.ensure(16 * sizeof(double)));
+  if (int rc = ensure_read(c)) return rc;
   return HEXOPT_OK;
 }
 
@@ -189,25 +219,31 @@ double tet_mass(const hexopt_params* prm) { return prm->tet_mass > 0 ? prm->tet_
 
 Cg64 cg64_buffers(hexopt_ctx* c) {
   Cg64 w{c->d_x.as<double>(), c->d_r.as<double>(), c->d_z.as<double>(), {c->d_p.as<double>(), c->d_p2.as<double>()},
-         c->d_tmp.as<double>(), c->d_halo.as<double>(), c->d_cg.p, {}};
+         c->d_tmp.as<double>(), c->d_halo.as<double>(), cg_state(c), {}};
   for (int i = 0; i < 8; ++i) w.part[i] = c->d_part[i].as<double>();
   return w;
 }
+
+struct EnergyParts {
+  double* p[4];
+  explicit EnergyParts(hexopt_ctx* c) {
+    for (int i = 0; i < 4; ++i) p[i] = c->d_part[i].as<double>();
+  }
+};
 
 int energy_now(hexopt_ctx* c, const hexopt_params* prm, const double* dst, double step, const double* aL, double* eq,
                double* es) {
   const int nsb = nblocks(c->sd.nb + c->sd.nC + c->sd.nT + c->sd.nL);
   double* out = c->d_scal.as<double>();
   launch_energy(refop(c), c->d_cur.as<double>(), dst, step, c->L.nV, c->tm.conn, c->L.nH, prm->energy, tet_mass(prm),
-                prm->exp_factor, c->sd, aL, c->d_part[0].as<double>(), c->d_part[1].as<double>(), nsb, out, c->stream);
-  double h[3] = {0, 0, 0};
+                prm->exp_factor, c->sd, aL, EnergyParts(c).p, nsb, out, nullptr, c->stream);
   if (c->glue)
     launch_glue_energy(soft_with(c, prm), c->L.nV, c->d_cur.as<double>(), dst, step, c->d_part[2].as<double>(), out + 2,
                        c->stream);
-  HIPCHK(c, hipMemcpyAsync(h, out, (c->glue ? 3 : 2) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  *eq = h[0];
-  *es = h[1] + h[2];
+  ReadBack rb;
+  if (int rc = read_back(c, rb)) return rc;
+  *eq = rb.scal[0];
+  *es = rb.scal[1] + (c->glue ? rb.scal[2] : 0.0);
   return HEXOPT_OK;
 }
 
@@ -300,6 +336,7 @@ void hexopt_destroy(hexopt_ctx* c) {
   if (!c) return;
   if (c->stream) { (void)hipStreamSynchronize(c->stream); }
   hipStream_t s = c->stream;
+  if (c->h_read) (void)hipHostFree(c->h_read);
   delete c;  // frees device buffers
   if (s) (void)hipStreamDestroy(s);
 }
@@ -345,14 +382,13 @@ int hexopt_reference(hexopt_ctx* c, const uint8_t* hflag, int cube) {
     dfl = c->d_hflag.as<uint8_t>();
   }
   HIPCHK(c, c->d_invs.ensure((size_t)8 * nH * sizeof(double) + 8));
-  HIPCHK(c, c->d_count.ensure(sizeof(int)));
-  HIPCHK(c, hipMemsetAsync(c->d_count.p, 0, sizeof(int), c->stream));
-  launch_ref_cube(c->d_rest.as<double>(), nV, c->tm.conn, nH, dfl, cube, c->d_invs.as<double>(), c->d_count.as<int>(),
+  if (ensure_read(c) != HEXOPT_OK) return HEXOPT_EHIP;
+  HIPCHK(c, hipMemsetAsync(counter(c), 0, sizeof(int), c->stream));
+  launch_ref_cube(c->d_rest.as<double>(), nV, c->tm.conn, nH, dfl, cube, c->d_invs.as<double>(), counter(c),
                   c->stream);
-  int ngen = 0;
-  HIPCHK(c, hipMemcpyAsync(&ngen, c->d_count.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (ngen == 0) {
+  ReadBack rb;
+  if (read_back(c, rb) != HEXOPT_OK) return HEXOPT_EHIP;
+  if (rb.count == 0) {
     c->ref_mode = REF_CUBE;
   } else {
     HIPCHK(c, c->d_B.ensure((size_t)72 * nH * sizeof(double) + 8));
@@ -547,7 +583,13 @@ int hexopt_slim_solve(hexopt_ctx* c, const hexopt_params* prm, int iters, hexopt
   if (nL > 0) HIPCHK(c, hipMemsetAsync(aL, 0, nL * sizeof(double), st));
   // slim_precompute: energy at the start point with a_L = 0
   double eq = 0, es = 0;
-  if ((rc = energy_now(c, prm, nullptr, 0.0, aL, &eq, &es)) != HEXOPT_OK) return rc;
+  const int nsb = nblocks(c->sd.nb + c->sd.nC + c->sd.nT + c->sd.nL);
+  if (c->glue || iters == 0) {
+    if ((rc = energy_now(c, prm, nullptr, 0.0, aL, &eq, &es)) != HEXOPT_OK) return rc;
+  } else {  // into scalars 8 and 9, read with the first line search
+    launch_energy(ro, c->d_cur.as<double>(), nullptr, 0.0, nV, c->tm.conn, nH, prm->energy, M, exp_f, c->sd, aL,
+                  EnergyParts(c).p, nsb, c->d_scal.as<double>() + 8, nullptr, st);
+  }
   double energy = (eq + es) / mesh_area;
   const int nb = nblocks(n);
   double* x = c->d_x.as<double>();
@@ -586,57 +628,59 @@ int hexopt_slim_solve(hexopt_ctx* c, const hexopt_params* prm, int iters, hexopt
       launch_apply(c->tm, ro, c->d_K.as<double>(), x, c->d_tmp.as<double>(), prox, sd, c->d_halo.as<double>(), pt, pf,
                    pl2, st);
       launch_cg_init(n, c->d_rhs.as<double>(), c->d_tmp.as<double>(), c->d_r.as<double>(), c->d_part[0].as<double>(),
-                     c->d_part[1].as<double>(), nb, c->d_cg.p, c->d_invd.as<double>(), c->d_p.as<double>(),
+                     c->d_part[1].as<double>(), nb, cg_state(c), c->d_invd.as<double>(), c->d_p.as<double>(),
                      c->d_part[5].as<double>(), 1e-8, st);
       for (int k = 0; k < 20; ++k) {
         launch_group_sum(sd, nV, c->d_p.as<double>(), gsum, st);
         launch_apply(c->tm, ro, c->d_K.as<double>(), c->d_p.as<double>(), c->d_tmp.as<double>(), prox, sd,
                      c->d_halo.as<double>(), pt, pf, pl2, st);
-        launch_cg_alpha(c->d_cg.p, pt, c->L.nTiles, pf, nfix, pl2, 0, st);
-        launch_cg_update(n, c->d_cg.p, x, c->d_r.as<double>(), c->d_z.as<double>(), c->d_p.as<double>(),
+        launch_cg_alpha(cg_state(c), pt, c->L.nTiles, pf, nfix, pl2, 0, st);
+        launch_cg_update(n, cg_state(c), x, c->d_r.as<double>(), c->d_z.as<double>(), c->d_p.as<double>(),
                          c->d_tmp.as<double>(), c->d_invd.as<double>(), c->d_part[6].as<double>(),
                          c->d_part[7].as<double>(), nb, c->d_p.as<double>(), st);
       }
     }
-    launch_cg_zero_if(n, c->d_cg.p, x, nb, st);
+    launch_cg_zero_if(n, cg_state(c), x, nb, st);
     if (c->glue) launch_glue_restore(nV, c->d_invd.as<double>(), cur, x, st);
     if (nL > 0 && !prm->projection)
       HIPCHK(c, hipMemcpyAsync(aL, x + 3 * (size_t)nV, nL * sizeof(double), hipMemcpyDeviceToDevice, st));
-    // flip-avoiding step bound and, outside the glue, the energy at the start of the line
-    // search, read back together
+    // flip-avoiding step bound and, outside the glue, the energies at the start of the line
+    // search and at its first step, read back together
     double* scal = c->d_scal.as<double>();
-    double q0 = 0, s0 = 0;
+    double q0 = 0, s0 = 0, q1 = 0, s1 = 0;
     launch_max_step(cur, x, nV, c->tm.conn, nH, c->d_part[0].as<double>(), scal + 4, st);
     if (!c->glue)
-      launch_energy(ro, cur, nullptr, 0.0, nV, c->tm.conn, nH, prm->energy, M, prm->exp_factor, c->sd, aL,
-                    c->d_part[0].as<double>(), c->d_part[1].as<double>(),
-                    nblocks(c->sd.nb + c->sd.nC + c->sd.nT + c->sd.nL), scal, st);
-    std::vector<unsigned char> cgs(cg_state_bytes());
-    double hs[5] = {0, 0, 0, 0, 0};
-    HIPCHK(c, hipMemcpyAsync(hs, scal, 5 * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipMemcpyAsync(cgs.data(), c->d_cg.p, cgs.size(), hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipStreamSynchronize(st));
-    const double tmin = hs[4];
+      launch_energy(ro, cur, x, 0.0, nV, c->tm.conn, nH, prm->energy, M, exp_f, c->sd, aL, EnergyParts(c).p, nsb, scal,
+                    scal + 4, st);
+    ReadBack rb;
+    if ((rc = read_back(c, rb)) != HEXOPT_OK) return rc;
+    const double tmin = rb.scal[4];
     int cg_iters = 0, cg_done = 0;
     double cg_err = 0;
-    read_cg_state(cgs.data(), &cg_iters, &cg_err, &cg_done);
+    read_cg_state(rb.cg, &cg_iters, &cg_err, &cg_done);
     double step = std::min(1., tmin * 0.8);
     const double bound = step;
     // igl::line_search (line_search.cpp:10-56)
     if (c->glue) {
       if ((rc = energy_now(c, prm, nullptr, 0.0, aL, &q0, &s0)) != HEXOPT_OK) return rc;
     } else {
-      q0 = hs[0];
-      s0 = hs[1];
+      q0 = rb.scal[0];
+      s0 = rb.scal[1];
+      q1 = rb.scal[2];
+      s1 = rb.scal[3];
+      if (it == 0) {
+        eq = rb.scal[8];
+        es = rb.scal[9];
+      }
     }
+    bool known = !c->glue;  // q1 and s1 are those of the step
     const double old_energy = q0 + s0;
     double new_energy = old_energy;
     int cur_iter = 0;
     while (new_energy >= old_energy) {
       if (cur_iter > 20) step = 0;
-      double q1, s1;
-      if ((rc = energy_now(c, prm, x, step, aL, &q1, &s1)) != HEXOPT_OK) return rc;
+      if (!known && (rc = energy_now(c, prm, x, step, aL, &q1, &s1)) != HEXOPT_OK) return rc;
+      known = false;
       const double cur_e = q1 + s1;
       eq = q1;
       es = s1;
@@ -829,8 +873,6 @@ static int ensure_state32(hexopt_ctx* c) {
   HIPCHK(c, c->f_halo.ensure(nh32 * sizeof(float)));
   HIPCHK(c, c->d_Ld64.ensure(n * sizeof(double)));
   HIPCHK(c, c->d_b64.ensure(n * sizeof(double)));
-  HIPCHK(c, c->d_ninv.ensure(sizeof(int)));
-  HIPCHK(c, c->d_cgsave.ensure(cg_state_bytes()));
   return HEXOPT_OK;
 }
 
@@ -846,18 +888,18 @@ static int cg32(hexopt_ctx* c, const SoftDev& sd, double prox, const float* b, f
   float* P[2] = {c->f_p.as<float>(), c->f_p2.as<float>()};
   float* z = c->f_z.as<float>();
   float* r = c->f_r.as<float>();
-  launch_cg32_init(nV, nL, sd, prox, b, c->f_invd.as<float>(), x, r, z, P[0], c->d_cg.p, c->d_part[0].as<double>(),
+  launch_cg32_init(nV, nL, sd, prox, b, c->f_invd.as<float>(), x, r, z, P[0], cg_state(c), c->d_part[0].as<double>(),
                    c->d_part[1].as<double>(), c->d_part[3].as<double>(), 1e-8, st);
   for (int k = 0; k < iters; ++k)
     launch_cg32_iteration(c->tm, ro, c->f_K.as<float>(), prox, sd, c->d_iso.as<int>(), c->n_iso, z,
                           P[k & 1], P[(k + 1) & 1], c->f_tmp.as<float>(), c->f_halo.as<float>(), c->f_invd.as<float>(),
-                          x, r, z, c->d_cg.p, c->d_part[2].as<double>(), c->d_part[4].as<double>(),
+                          x, r, z, cg_state(c), c->d_part[2].as<double>(), c->d_part[4].as<double>(),
                           c->d_part[5].as<double>(), c->d_part[3].as<double>(), c->d_part[6].as<double>(),
                           c->d_part[7].as<double>(), k, k == iters - 1, st);
   HIPCHK(c, hipGetLastError());
   if (it_out || err_out) {
     std::vector<unsigned char> cgs(cg_state_bytes());
-    HIPCHK(c, hipMemcpyAsync(cgs.data(), c->d_cg.p, cgs.size(), hipMemcpyDeviceToHost, st));
+    HIPCHK(c, hipMemcpyAsync(cgs.data(), cg_state(c), cgs.size(), hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipStreamSynchronize(st));
     int done = 0, its = 0;
     double err = 0;
@@ -894,13 +936,13 @@ int hexopt_opt32_solve(hexopt_ctx* c, const hexopt_params* prm, const hexopt_opt
   double energy = 0;
   for (int it = 0; it < iters; ++it) {
     // one pass over the elements: energy, adjoint rhs -dE/dx/2, K, Jacobi diagonal
-    HIPCHK(c, hipMemsetAsync(c->d_ninv.p, 0, sizeof(int), st));
+    HIPCHK(c, hipMemsetAsync(counter(c), 0, sizeof(int), st));
     launch_adj_local32(c->tm, ro, cur, c->f_K.as<float>(), M, prox, sd, c->f_rhs.as<float>(), c->f_invd.as<float>(),
-                       c->f_halo.as<float>(), c->d_ninv.as<int>(), st);
+                       c->f_halo.as<float>(), counter(c), st);
     // direction: L d = -dE/dx / 2 by FP32 CG, then one FP64-residual refinement solve
     float* d = c->f_d.as<float>();
     if ((rc = cg32(c, sd, prox, c->f_rhs.as<float>(), d, opt->cg_iters, nullptr, nullptr))) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->d_cgsave.p, c->d_cg.p, cg_state_bytes(), hipMemcpyDeviceToDevice, st));
+    HIPCHK(c, hipMemcpyAsync(cg_saved(c), cg_state(c), cg_state_bytes(), hipMemcpyDeviceToDevice, st));
     const int nb = nblocks(n);
     const bool every = opt->residual_every > 0 && (it % opt->residual_every == 0 || it == iters - 1);
     const bool measure = opt->refine_iters > 0 || every;
@@ -936,35 +978,33 @@ int hexopt_opt32_solve(hexopt_ctx* c, const hexopt_params* prm, const hexopt_opt
     // FP64 flip-free bound, then the reference's bisection on FP64 energies along the FP32
     // direction
     launch_max_step_dir32(cur, d, nV, c->tm.conn, nH, c->d_part[0].as<double>(), scal + 4, st);
-    launch_energy_dir32(ro, cur, d, 0.0, nV, c->tm.conn, nH, M, sd, aL, c->d_part[0].as<double>(),
-                        c->d_part[1].as<double>(), nsb, scal, st);
-    double hs[10];
-    int ninv = 0;
-    std::vector<unsigned char> cgs(cg_state_bytes());
-    HIPCHK(c, hipMemcpyAsync(hs, scal, 10 * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipMemcpyAsync(&ninv, c->d_ninv.p, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipMemcpyAsync(cgs.data(), c->d_cgsave.p, cgs.size(), hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipStreamSynchronize(st));
+    launch_energy_dir32(ro, cur, d, 0.0, nV, c->tm.conn, nH, M, sd, aL, EnergyParts(c).p, nsb, scal, scal + 4, st);
+    ReadBack rb;
+    if ((rc = read_back(c, rb))) return rc;
+    const int ninv = rb.count;
+    const double* hs = rb.scal;
     int cg_it = 0, cg_done = 0;
     double cg_err = 0;
-    read_cg_state(cgs.data(), &cg_it, &cg_err, &cg_done);
+    read_cg_state(rb.saved, &cg_it, &cg_err, &cg_done);
     // |b64| of the direction system, from the FP64 right-hand side
     const double rhs_norm = std::sqrt(hs[7]);
     const double res64 = hs[6];
     const double tmin = hs[4];
-    double h2[2] = {hs[0], hs[1]};
-    const double old_energy = h2[0] + h2[1];
+    const double refined64 = hs[8];
+    const double old_energy = hs[0] + hs[1];
     double step = std::min(1., tmin * 0.8);
     const double bound = step;
-    double new_energy = old_energy, eq = h2[0], es = h2[1];
+    double new_energy = old_energy, eq = hs[0], es = hs[1];
+    double h2[2] = {hs[2], hs[3]};  // the energies of the first step
     int cur_iter = 0;
     while (new_energy >= old_energy) {
       if (cur_iter > 20) step = 0;
-      launch_energy_dir32(ro, cur, d, step, nV, c->tm.conn, nH, M, sd, aL, c->d_part[0].as<double>(),
-                          c->d_part[1].as<double>(), nsb, scal, st);
-      HIPCHK(c, hipMemcpyAsync(h2, scal, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-      HIPCHK(c, hipStreamSynchronize(st));
+      if (cur_iter > 0) {
+        launch_energy_dir32(ro, cur, d, step, nV, c->tm.conn, nH, M, sd, aL, EnergyParts(c).p, nsb, scal, nullptr, st);
+        if ((rc = read_back(c, rb))) return rc;
+        h2[0] = rb.scal[0];
+        h2[1] = rb.scal[1];
+      }
       const double ce = h2[0] + h2[1];
       if (std::isnan(ce) || std::isinf(ce) || ce > old_energy) {
         step /= 2;
@@ -985,7 +1025,7 @@ int hexopt_opt32_solve(hexopt_ctx* c, const hexopt_params* prm, const hexopt_opt
       lg.cg_iters = cg_it; lg.cg_error = cg_err;
       lg.residual64 = !measure ? -1.0 : (rhs_norm > 0 ? std::sqrt(res64) / rhs_norm : 0.0);
       lg.residual64_refined = !(every && opt->refine_iters > 0) ? -1.0
-                              : (rhs_norm > 0 ? std::sqrt(hs[8]) / rhs_norm : 0.0);
+                              : (rhs_norm > 0 ? std::sqrt(refined64) / rhs_norm : 0.0);
       lg.inverted_tets = ninv;
     }
   }
@@ -1015,9 +1055,9 @@ int hexopt_debug_operator(hexopt_ctx* c, const hexopt_params* prm, int precision
     K64.resize((size_t)48 * nH);
     HIPCHK(c, hipMemcpyAsync(K64.data(), c->d_K.p, K64.size() * 8, hipMemcpyDeviceToHost, st));
   } else {
-    HIPCHK(c, hipMemsetAsync(c->d_ninv.p, 0, sizeof(int), st));
+    HIPCHK(c, hipMemsetAsync(counter(c), 0, sizeof(int), st));
     launch_adj_local32(c->tm, refop(c), c->d_cur.as<double>(), c->f_K.as<float>(), M, prox, sd, c->f_rhs.as<float>(),
-                       c->f_invd.as<float>(), c->f_halo.as<float>(), c->d_ninv.as<int>(), st);
+                       c->f_invd.as<float>(), c->f_halo.as<float>(), counter(c), st);
     K32.resize((size_t)48 * nH);
     HIPCHK(c, hipMemcpyAsync(K32.data(), c->f_K.p, K32.size() * 4, hipMemcpyDeviceToHost, st));
   }
@@ -1057,7 +1097,7 @@ int hexopt_time_kernel(hexopt_ctx* c, int which, int reps, double* ms_per_launch
         // the update partials of the last solve (a zero threshold keeps every pass running)
         (void)launch_cg32_apply_folded(c->tm, ro, c->f_K.as<float>(), sd, c->d_iso.as<int>(), c->n_iso,
                                        c->f_z.as<float>(), c->f_p.as<float>(), c->f_p2.as<float>(),
-                                       c->f_tmp.as<float>(), c->f_halo.as<float>(), c->d_cg.p,
+                                       c->f_tmp.as<float>(), c->f_halo.as<float>(), cg_state(c),
                                        c->d_part[2].as<double>(), c->d_part[4].as<double>(),
                                        c->d_part[5].as<double>(), c->d_part[3].as<double>(),
                                        c->d_part[6].as<double>(), c->d_part[7].as<double>(), 0, st);
@@ -1076,7 +1116,7 @@ int hexopt_time_kernel(hexopt_ctx* c, int which, int reps, double* ms_per_launch
         break;
       default:
         launch_adj_local32(tm, ro, c->d_cur.as<double>(), c->f_K.as<float>(), 1.0, 1e-5, sd, c->f_rhs.as<float>(),
-                           c->f_invd.as<float>(), c->f_halo.as<float>(), c->d_ninv.as<int>(), st);
+                           c->f_invd.as<float>(), c->f_halo.as<float>(), counter(c), st);
     }
   };
   sd.nL = 0;
@@ -1087,9 +1127,9 @@ int hexopt_time_kernel(hexopt_ctx* c, int which, int reps, double* ms_per_launch
   }
   if (which == 1) {
     // a fresh CG state (not converged) on the current FP32 system, so the pass runs in full
-    HIPCHK(c, hipMemsetAsync(c->d_cg.p, 0, cg_state_bytes(), st));
+    HIPCHK(c, hipMemsetAsync(cg_state(c), 0, cg_state_bytes(), st));
     launch_cg32_init(c->L.nV, c->nL, sd, 1e-5, c->f_rhs.as<float>(), c->f_invd.as<float>(), c->f_d.as<float>(),
-                     c->f_r.as<float>(), c->f_z.as<float>(), c->f_p.as<float>(), c->d_cg.p, c->d_part[0].as<double>(),
+                     c->f_r.as<float>(), c->f_z.as<float>(), c->f_p.as<float>(), cg_state(c), c->d_part[0].as<double>(),
                      c->d_part[1].as<double>(), c->d_part[3].as<double>(), 0.0, st);
   }
   one();  // warm

@@ -100,9 +100,12 @@ size_t cg_state_bytes();
 void read_cg_state(const void* host_state, int* iters, double* tol_error, int* done);
 void launch_max_step(const double* cur, const double* dst, int nV, const int* conn, int nH, double* part, double* out,
                      hipStream_t st);
+// (quality, soft) energy of cur + step (dst - cur) into out[0..1], partials in part[0..1]. With
+// tmin: of cur into out[0..1] and of the first step a line search takes for the bound *tmin into
+// out[2..3] (step is not read, part[2..3] hold the second partials)
 void launch_energy(const RefOp& ro, const double* cur, const double* dst, double step, int nV, const int* conn, int nH,
-                   int energy, double M, double exp_f, const SoftDev& sd, const double* aL, double* part_q,
-                   double* part_s, int ns_blocks, double* out2, hipStream_t st);
+                   int energy, double M, double exp_f, const SoftDev& sd, const double* aL, double* const* part,
+                   int ns_blocks, double* out, const double* tmin, hipStream_t st);
 void launch_step(int n, double* cur, const double* dst, double step, hipStream_t st);
 void launch_grad(int prec, const TileMesh& tm, const RefOp& ro, const void* X, void* G, double M, const SoftDev& sd,
                  const double* aL, void* halo, hipStream_t st);
@@ -171,8 +174,8 @@ void launch_add_inplace(int n, float* d, const float* e, int nb, hipStream_t st)
 void launch_max_step_dir32(const double* cur, const float* d, int nV, const int* conn, int nH, double* part,
                            double* out, hipStream_t st);
 void launch_energy_dir32(const RefOp& ro, const double* cur, const float* d, double step, int nV, const int* conn,
-                         int nH, double M, const SoftDev& sd, const double* aL, double* part_q, double* part_s,
-                         int ns_blocks, double* out2, hipStream_t st);
+                         int nH, double M, const SoftDev& sd, const double* aL, double* const* part, int ns_blocks,
+                         double* out, const double* tmin, hipStream_t st);
 void launch_step_dir32(int n, double* cur, const float* d, double step, hipStream_t st);
 void launch_sum_partials(const double* part, int n, double* out, hipStream_t st);
 
