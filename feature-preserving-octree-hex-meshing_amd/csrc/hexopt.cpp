@@ -938,7 +938,7 @@ int hexopt_opt32_solve(hexopt_ctx* c, const hexopt_params* prm, const hexopt_opt
     // one pass over the elements: energy, adjoint rhs -dE/dx/2, K, Jacobi diagonal
     HIPCHK(c, hipMemsetAsync(counter(c), 0, sizeof(int), st));
     launch_adj_local32(c->tm, ro, cur, c->f_K.as<float>(), M, prox, sd, c->f_rhs.as<float>(), c->f_invd.as<float>(),
-                       c->f_halo.as<float>(), counter(c), st);
+                       c->f_halo.as<float>(), c->d_part[0].as<double>(), counter(c), st);
     // direction: L d = -dE/dx / 2 by FP32 CG, then one FP64-residual refinement solve
     float* d = c->f_d.as<float>();
     if ((rc = cg32(c, sd, prox, c->f_rhs.as<float>(), d, opt->cg_iters, nullptr, nullptr))) return rc;
@@ -1057,7 +1057,8 @@ int hexopt_debug_operator(hexopt_ctx* c, const hexopt_params* prm, int precision
   } else {
     HIPCHK(c, hipMemsetAsync(counter(c), 0, sizeof(int), st));
     launch_adj_local32(c->tm, refop(c), c->d_cur.as<double>(), c->f_K.as<float>(), M, prox, sd, c->f_rhs.as<float>(),
-                       c->f_invd.as<float>(), c->f_halo.as<float>(), counter(c), st);
+                       c->f_invd.as<float>(), c->f_halo.as<float>(), c->d_part[0].as<double>(), counter(c),
+                       st);
     K32.resize((size_t)48 * nH);
     HIPCHK(c, hipMemcpyAsync(K32.data(), c->f_K.p, K32.size() * 4, hipMemcpyDeviceToHost, st));
   }
@@ -1116,7 +1117,8 @@ int hexopt_time_kernel(hexopt_ctx* c, int which, int reps, double* ms_per_launch
         break;
       default:
         launch_adj_local32(tm, ro, c->d_cur.as<double>(), c->f_K.as<float>(), 1.0, 1e-5, sd, c->f_rhs.as<float>(),
-                           c->f_invd.as<float>(), c->f_halo.as<float>(), counter(c), st);
+                           c->f_invd.as<float>(), c->f_halo.as<float>(), c->d_part[0].as<double>(),
+                           counter(c), st);
     }
   };
   sd.nL = 0;

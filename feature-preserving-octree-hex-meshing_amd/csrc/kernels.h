@@ -113,7 +113,8 @@ void launch_hvp(int prec, const TileMesh& tm, const RefOp& ro, const void* X, co
                 const SoftDev& sd, void* halo, hipStream_t st);
 // FP32 optimiser (adjoint formulation of the SLIM step)
 void launch_adj_local32(const TileMesh& tm, const RefOp& ro, const double* X, float* K, double M, double prox,
-                        const SoftDev& sd, float* rhs, float* invd, float* halo, int* n_inverted, hipStream_t st);
+                         const SoftDev& sd, float* rhs, float* invd, float* halo, double* hex_part, int* n_inverted,
+                         hipStream_t st);
 void launch_apply32_f64(const TileMesh& tm, const RefOp& ro, const float* K, const float* p, double* out, double prox,
                         const SoftDev& sd, double* halo, hipStream_t st);
 // Fused FP32 CG (Eigen's algorithm, FP64 dot products) on the CG operator:

@@ -285,7 +285,8 @@ __device__ __forceinline__ void scatter_tile4(const TileMesh& tm, int tile, int 
 
 // ---------------------------------------------------------------------------------------
 // Tiled scatter skeleton. Op provides:
-//   __device__ void hex(int h, T out[8][NC])          per-hex corner contributions
+//   __device__ double hex(int h, T out[8][NC])        per-hex corner contributions; returns
+//                                                       the hex's share of an optional sum
 //   __device__ double finish(int v, T acc[NC])        writes vertex v; returns its share of
 //                                                       the kernel's optional vertex sum
 // minimum waves per SIMD the register allocation of a tile pass must leave room for (1: no
@@ -297,7 +298,7 @@ struct TileWaves {
 
 template <class T, int NC, class Op>
 __global__ __launch_bounds__(kTileHex) __attribute__((amdgpu_waves_per_eu(TileWaves<Op>::value)))
-void tile_scatter_kernel(TileMesh tm, Op op, T* halo, double* partial) {
+void tile_scatter_kernel(TileMesh tm, Op op, T* halo, double* partial, double* hex_partial) {
   __shared__ T acc[NC * kMaxLV];
   __shared__ double red[16];
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -308,13 +309,18 @@ void tile_scatter_kernel(TileMesh tm, Op op, T* halo, double* partial) {
   T c[8][NC];
   int li[8];
   const bool active = tid < nh;
+  double hv = 0.0;
 #pragma unroll
   for (int k = 0; k < 8; ++k)
 #pragma unroll
     for (int j = 0; j < NC; ++j) c[k][j] = T(0);
   if (active) {
-    op.hex(h0 + tid, c);
+    hv = op.hex(h0 + tid, c);
     load_li(tm, h0 + tid, li);
+  }
+  if (hex_partial) {
+    double sh = block_sum(hv, red);
+    if (tid == 0) hex_partial[tile] = sh;
   }
   __syncthreads();
   scatter_tile<T, NC>(tm, tile, tm.tile_corner[tile], nh, active, li, c, acc);
@@ -361,9 +367,11 @@ __global__ __launch_bounds__(256) void fixup_kernel(TileMesh tm, Op op, const T*
 }
 
 template <class T, int NC, class Op>
-void launch_scatter(const TileMesh& tm, const Op& op, T* halo, double* part_tile, double* part_fix, hipStream_t st) {
+void launch_scatter(const TileMesh& tm, const Op& op, T* halo, double* part_tile, double* part_fix, hipStream_t st,
+                    double* hex_part = nullptr) {
   if (tm.nTiles > 0)
-    hipLaunchKernelGGL((tile_scatter_kernel<T, NC, Op>), dim3(tm.nTiles), dim3(kTileHex), 0, st, tm, op, halo, part_tile);
+    hipLaunchKernelGGL((tile_scatter_kernel<T, NC, Op>), dim3(tm.nTiles), dim3(kTileHex), 0, st, tm, op, halo, part_tile,
+                       hex_part);
   if (tm.nShared > 0)
     hipLaunchKernelGGL((fixup_kernel<T, NC, Op>), dim3((tm.nShared + 255) / 256), dim3(256), 0, st, tm, op,
                        (const T*)halo, part_fix);
@@ -653,7 +661,7 @@ struct LocalStepOp {
         for (int d = 0; d < 3; ++d) out[tc[k + 1]][3 + d] += Kt[d][d] * nk[k];
     }
   }
-  __device__ void hex(int h, double out[8][6]) const {
+  __device__ double hex(int h, double out[8][6]) const {
     int vid[8];
     double p[8][3];
     gather8(X, nV, conn, nH, h, vid, p);
@@ -669,6 +677,7 @@ struct LocalStepOp {
       rotate_rings(p);
       rotate_rings(out);
     }
+    return 0.0;
   }
   __device__ double finish(int g, double acc[6]) const {
     double dg[3] = {acc[3] + prox, acc[4] + prox, acc[5] + prox};
@@ -798,7 +807,7 @@ struct LocalStepCubeOp : LocalStepOp<true> {
     }
     add_row<3, 3>(out, kHexTet[c][0], k3);
   }
-  __device__ void hex(int h, double out[8][6]) const {
+  __device__ double hex(int h, double out[8][6]) const {
     unsigned left = 0;
     {
       int vid[8];
@@ -818,6 +827,7 @@ struct LocalStepCubeOp : LocalStepOp<true> {
 #pragma unroll 1
     for (int c = 0; c < 8; ++c)
       if ((left >> c) & 1) svd_tet(h, c, out);
+    return 0.0;
   }
 };
 
@@ -881,7 +891,7 @@ template <class KT, class PT, class CT, class OT>
 struct ApplyOp {
   RefOp ro; int nV, nH; const int* conn; const KT* K; const PT* p; OT* out; double prox;
   SoftDev sd; const PT* pa; int nL;
-  __device__ void hex(int h, CT o[8][3]) const {
+  __device__ double hex(int h, CT o[8][3]) const {
     CT q[8][3];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -890,6 +900,7 @@ struct ApplyOp {
       for (int d = 0; d < 3; ++d) q[k][d] = (CT)p[(size_t)d * nV + v];
     }
     hex_forces<KT, CT>(ro, K, nH, h, q, o);
+    return 0.0;
   }
   __device__ double finish(int g, CT acc[3]) const {
     double pv[3] = {(double)p[g], (double)p[(size_t)nV + g], (double)p[2 * (size_t)nV + g]};
@@ -916,32 +927,18 @@ struct ApplyOp {
 
 // ---------------------------------------------------------------------------------------
 // FP32 adjoint + local step of the symmetric-Dirichlet energy (the FP32 optimiser's only
-// pass over the elements per iteration): per corner tet the SLIM weights K = M W^T W and
-// dE/dJ, formed in FP64 from the FP64 corners and rounded once (K stored FP32); scatters the
-// direction rhs -dE/dx / 2 and the Jacobi diagonal in FP32 and counts the inverted tets. FP64
-// costs no more than unpacked FP32 here (the vector units run both at one rate), and it needs
-// none of the special forms that FP32 wants near a rotation: there W, dE/dJ = 2 (J - T^3 Q)
-// and the m = 1 band |s - 1| < 1e-8 come out to FP64's precision (sd_polar).
-__device__ __forceinline__ void sd_adjoint(const double J[3][3], const double Q[3][3], const double T3[6],
-                                           double P[3][3]) {
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    P[0][k] = J[0][k] - (T3[0] * Q[0][k] + T3[3] * Q[1][k] + T3[4] * Q[2][k]);
-    P[1][k] = J[1][k] - (T3[3] * Q[0][k] + T3[1] * Q[1][k] + T3[5] * Q[2][k]);
-    P[2][k] = J[2][k] - (T3[4] * Q[0][k] + T3[5] * Q[1][k] + T3[2] * Q[2][k]);
-  }
-}
-
-// W^2 and half of dE/dJ by the SVD, for the tets that sd_polar leaves to it
-__device__ __forceinline__ void sd_adjoint_svd(const double J[3][3], double W2[6], double P[3][3]) {
-  double R[3][3];
-  sd_svd(J, W2, R);
-  (void)sd_energy_grad(J, P);
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) P[i][j] *= 0.5;
-}
+// pass over the elements per iteration): per corner tet in FP32 arithmetic the Jacobian,
+// its SVD, the SLIM weights K = M W^T W (stored FP32), the energy, and dE/dJ; scatters the
+// direction rhs -dE/dx / 2 and the Jacobi diagonal. The corner-determinant sign is tested
+// in FP64 (inverted-tet count); the energy is summed in FP64.
+struct AdjLocalOp32;
+// three waves per SIMD: the FP64 corners and the hex's 8 x 6 sums stay live through the
+// corner-tet loops; 37 values spill, and it still runs faster than two waves without spills
+// (415 against 420 us on the 1.1M-hex octree torus)
+template <>
+struct TileWaves<AdjLocalOp32> {
+  static constexpr int value = 3;
+};
 
 struct AdjLocalOp32 {
   RefOp ro; int nV, nH; const int* conn; const double* X; float* K; double M, prox;
@@ -949,60 +946,103 @@ struct AdjLocalOp32 {
 
   // Corner tet c whose corners are rows T0, T1, T2, T3 of pd / out (compile-time indices: the
   // caller rotates the rows so that every corner tet of a ring takes the same four rows).
+  // Per tet, FP64 first: the Jacobian J = E B from the FP64 corners, its orientation (sign of
+  // det J; for a cube reference B = invs * (a permutation with determinant +1 for every
+  // corner) and invs > 0, so the sign is that of det E), and its deviation from isometry
+  // D = J J^T - I. Then FP32 for the rest: the weights (the reference's m = 1 branch,
+  // |s_i - 1| < 1e-8 (slim_m.cpp:351-353), is taken for the tet when |D|_F < 2e-8 puts every
+  // singular value inside it, a threshold FP32 cannot resolve), and the energy and dE/dJ in
+  // their deviation form, which keeps FP32's relative precision where J is near a rotation.
   template <int T0, int T1, int T2, int T3>
-  __device__ __forceinline__ void tet(int h, int c, const double pd[8][3], float out[8][6], int& inv) const {
+  __device__ __forceinline__ void tet(int h, int c, const double pd[8][3], float out[8][6], double& e, int& inv) const {
     constexpr int tc[4] = {T0, T1, T2, T3};
-    double E[3][3], B[3][3], J[3][3], W2[6], P[3][3];
+    double E64[3][3], B64[3][3], J64[3][3], D64[3][3];
 #pragma unroll
     for (int k = 0; k < 3; ++k)
 #pragma unroll
-      for (int d = 0; d < 3; ++d) E[d][k] = pd[tc[k + 1]][d] - pd[T0][d];
-    tet_B(ro, nH, h, c, B);
-    matmul3(E, B, J);
-    inv += det3(J) < 0.0;
-    double Q[3][3], cube[6];
-    if (sd_polar(J, 1.0, Q, W2, cube)) sd_adjoint(J, Q, cube, P);
-    else sd_adjoint_svd(J, W2, P);
+      for (int d = 0; d < 3; ++d) E64[d][k] = pd[tc[k + 1]][d] - pd[T0][d];
+    tet_B(ro, nH, h, c, B64);
+    matmul3(E64, B64, J64);
+    inv += (ro.mode == REF_CUBE ? det3(E64) : det3(J64)) < 0.0;
+    const double dev2 = isometry_deviation(J64, D64);
+    const bool iso = dev2 < 4e-16;
+    float B[3][3], J[3][3], D[3][3], W[3][3], P[3][3];
 #pragma unroll
-    for (int j = 0; j < 6; ++j) K[k_at<float>(c * 6 + j, h, nH)] = (float)(M * W2[j]);
-    // -dE/dx / 2 of the tet's corners: row k + 1 gets P B_k, row 0 minus their sum; and the
-    // Jacobi diagonal
-    const double g0[3] = {B[0][0] + B[1][0] + B[2][0], B[0][1] + B[1][1] + B[2][1], B[0][2] + B[1][2] + B[2][2]};
-    const double n0 = g0[0] * g0[0] + g0[1] * g0[1] + g0[2] * g0[2];
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j2 = 0; j2 < 3; ++j2) {
+        B[i][j2] = (float)B64[i][j2];
+        J[i][j2] = (float)J64[i][j2];
+        D[i][j2] = (float)D64[i][j2];
+      }
+    if (iso) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j2 = 0; j2 < 3; ++j2) W[i][j2] = i == j2 ? 1.0f : 0.0f;
+    } else {
+      slim_weights_sd_stable(J, W);
+    }
+    // the deviation form while I + D is well conditioned (|D|_F < 0.5); the direct form
+    // else, where inverting J J^T would square J's condition number
+    if (dev2 < 0.25) e += M * (6.0 + (double)sd_energy_grad_dev(J, D, P));
+    else e += M * (double)sd_energy_grad(J, P);
+    float Kt[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) Kt[i][j] = (float)M * (W[0][i] * W[0][j] + W[1][i] * W[1][j] + W[2][i] * W[2][j]);
+    float s2 = 1.0f;
+    if (ro.mode == REF_CUBE) { float sc = (float)ro.invs[(size_t)c * nH + h]; s2 = sc * sc; }
+    const float ks[6] = {Kt[0][0], Kt[1][1], Kt[2][2], Kt[0][1], Kt[0][2], Kt[1][2]};
+#pragma unroll
+    for (int j = 0; j < 6; ++j) K[k_at<float>(c * 6 + j, h, nH)] = ks[j] * s2;
+    // -dE/dx / 2 of the tet's corners: row k + 1 gets P B_k, row 0 minus their sum
+    const float hm = -0.5f * (float)M;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const double nk = B[k][0] * B[k][0] + B[k][1] * B[k][1] + B[k][2] * B[k][2];
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const float f = (float)(-M * (P[d][0] * B[k][0] + P[d][1] * B[k][1] + P[d][2] * B[k][2]));
+        const float f = hm * (P[d][0] * B[k][0] + P[d][1] * B[k][1] + P[d][2] * B[k][2]);
         out[tc[k + 1]][d] += f;
         out[T0][d] -= f;
-        out[tc[k + 1]][3 + d] += (float)(M * W2[d] * nk);
       }
     }
+    // Jacobi diagonal
+    const float g0[3] = {-(B[0][0] + B[1][0] + B[2][0]), -(B[0][1] + B[1][1] + B[2][1]),
+                         -(B[0][2] + B[1][2] + B[2][2])};
+    const float n0 = g0[0] * g0[0] + g0[1] * g0[1] + g0[2] * g0[2];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) out[T0][3 + d] += (float)(M * W2[d] * n0);
+    for (int d = 0; d < 3; ++d) out[T0][3 + d] += Kt[d][d] * n0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float nk = B[k][0] * B[k][0] + B[k][1] * B[k][1] + B[k][2] * B[k][2];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) out[tc[k + 1]][3 + d] += Kt[d][d] * nk;
+    }
   }
 
-  __device__ void hex(int h, float out[8][6]) const {
+  __device__ double hex(int h, float out[8][6]) const {
     int vid[8];
     double pd[8][3];
     gather8(X, nV, conn, nH, h, vid, pd);
+    double e = 0.0;
     int inv = 0;
     // the ring's first tet pattern on rows turned r steps is tet r (rotate_rings)
 #pragma unroll 1
     for (int r = 0; r < 4; ++r) {
-      tet<0, 3, 4, 1>(h, r, pd, out, inv);
+      tet<0, 3, 4, 1>(h, r, pd, out, e, inv);
       rotate_rings(pd);
       rotate_rings(out);
     }
 #pragma unroll 1
     for (int r = 0; r < 4; ++r) {
-      tet<4, 7, 5, 0>(h, 4 + r, pd, out, inv);
+      tet<4, 7, 5, 0>(h, 4 + r, pd, out, e, inv);
       rotate_rings(pd);
       rotate_rings(out);
     }
     if (inv) atomicAdd(n_inverted, inv);
+    return e;
   }
   __device__ double finish(int g, float acc[6]) const {
     double dg[3] = {(double)acc[3] + prox, (double)acc[4] + prox, (double)acc[5] + prox};
@@ -1025,115 +1065,6 @@ struct AdjLocalOp32 {
     }
     return 0.0;
   }
-};
-
-// The same on cube references, laid out as LocalStepCubeOp: edges scaled by invs instead of an
-// operator B, a ring's four tets unrolled, the SVD's tets after them.
-struct AdjLocalCubeOp32 : AdjLocalOp32 {
-  __device__ __forceinline__ void store_K(int h, int c, const float ks[6]) const {
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      *reinterpret_cast<float2*>(K + k_at<float>(c * 6 + 2 * j, h, nH)) = make_float2(ks[2 * j], ks[2 * j + 1]);
-  }
-  // false: nothing added, the tet is left to svd_tet
-  template <int R0>
-  __device__ __forceinline__ bool cube_tet(int h, int c, double sg, const double p[8][3], float out[8][6],
-                                           int& inv) const {
-    constexpr int tc[3] = {(R0 + 3) & 3, R0 + 4, (R0 + 1) & 3};
-    const double s = ro.invs[(size_t)c * nH + h];
-    double J[3][3], W2[6], cube[6], Q[3][3], P[3][3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) J[d][k] = s * (p[tc[k]][d] - p[R0][d]);
-    if (!sd_polar(J, sg, Q, W2, cube)) return false;
-    inv += s < 0.0;  // det J > 0: the edges are mirrored where the rest tet (and so invs) was
-    sd_adjoint(J, Q, cube, P);
-    const double ms = -M * s, ms2 = M * s * s;
-    float ks[6];
-#pragma unroll
-    for (int j = 0; j < 6; ++j) ks[j] = (float)(ms2 * W2[j]);
-    store_K(h, c, ks);
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const float f = (float)(ms * P[d][k]);
-        out[tc[k]][d] += f;
-        out[R0][d] -= f;
-        out[tc[k]][3 + d] += ks[d];
-      }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) out[R0][3 + d] += 3.0f * ks[d];
-    return true;
-  }
-  __device__ __forceinline__ void svd_tet(int h, int c, float out[8][6], int& inv) const {
-    const double s = ro.invs[(size_t)c * nH + h];
-    double J[3][3], W2[6], P[3][3], x0[3];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int v = conn[(size_t)kHexTet[c][k] * nH + h];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double x = X[(size_t)d * nV + v];
-        if (k == 0) x0[d] = x;
-        else J[d][k - 1] = s * (x - x0[d]);
-      }
-    }
-    inv += s < 0.0 ? det3(J) > 0.0 : det3(J) < 0.0;
-    sd_adjoint_svd(J, W2, P);
-    const double ms = -M * s, ms2 = M * s * s;
-    float ks[6], k3[3];
-#pragma unroll
-    for (int j = 0; j < 6; ++j) ks[j] = (float)(ms2 * W2[j]);
-    store_K(h, c, ks);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const float f[3] = {(float)(ms * P[0][k]), (float)(ms * P[1][k]), (float)(ms * P[2][k])};
-      const float mf[3] = {-f[0], -f[1], -f[2]};
-      add_row<0, 3>(out, kHexTet[c][k + 1], f);
-      add_row<0, 3>(out, kHexTet[c][0], mf);
-      add_row<3, 3>(out, kHexTet[c][k + 1], ks);
-      k3[k] = 3.0f * ks[k];
-    }
-    add_row<3, 3>(out, kHexTet[c][0], k3);
-  }
-  __device__ void hex(int h, float out[8][6]) const {
-    unsigned left = 0;
-    int inv = 0;
-    {
-      int vid[8];
-      double p[8][3];
-      gather8(X, nV, conn, nH, h, vid, p);
-#pragma unroll 1
-      for (int c = 0; c < 8; c += 4) {
-        const double sg = c == 0 ? 1.0 : -1.0;
-        left |= (unsigned)!cube_tet<0>(h, c, sg, p, out, inv) << c;
-        left |= (unsigned)!cube_tet<1>(h, c + 1, sg, p, out, inv) << (c + 1);
-        left |= (unsigned)!cube_tet<2>(h, c + 2, sg, p, out, inv) << (c + 2);
-        left |= (unsigned)!cube_tet<3>(h, c + 3, sg, p, out, inv) << (c + 3);
-        swap_rings(p);
-        swap_rings(out);
-      }
-    }
-#pragma unroll 1
-    for (int c = 0; c < 8; ++c)
-      if ((left >> c) & 1) svd_tet(h, c, out, inv);
-    if (inv) atomicAdd(n_inverted, inv);
-  }
-};
-
-// VALU-bound: 410 us with the FP32 SVD and deviation forms (three waves per SIMD, 37 spills),
-// 291-317 us in this form at two waves (213 registers), 361 us at three with spills, per pass on
-// the 1.1M-hex octree torus. The positions after two iterations there are 2.7e-8 off a 64-bit
-// solve with the former weights, 3.7e-9 with these.
-template <>
-struct TileWaves<AdjLocalOp32> {
-  static constexpr int value = 2;
-};
-template <>
-struct TileWaves<AdjLocalCubeOp32> {
-  static constexpr int value = 2;
 };
 
 // rhs of the a_L rows of the direction system at a_L = 0: lamL t . (x_v - o)
@@ -2608,7 +2539,7 @@ struct GradOp {
       for (int d = 0; d < 3; ++d) o[T0][d] += -f[d];
     }
   }
-  __device__ void hex(int h, T o[8][3]) const {
+  __device__ double hex(int h, T o[8][3]) const {
     int vid[8];
     double pd[8][3];
     gather8(X, nV, conn, nH, h, vid, pd);
@@ -2625,6 +2556,7 @@ struct GradOp {
       rotate_rings(pd);
       rotate_rings(o);
     }
+    return e;
   }
   // soft gradient 2 (S x - b - lamL a t) for constrained vertices
   __device__ double finish(int g, T acc[3]) const {
@@ -2649,7 +2581,7 @@ struct GradOp {
 template <class T, class P>
 struct HvpOp {
   RefOp ro; int nV, nH; const int* conn; const P* X; const P* Vd; P* Hv; double M; SoftDev sd;
-  __device__ void hex(int h, T o[8][3]) const {
+  __device__ double hex(int h, T o[8][3]) const {
     int vid[8];
     double pd[8][3], vd[8][3];
     gather8(X, nV, conn, nH, h, vid, pd);
@@ -2670,6 +2602,7 @@ struct HvpOp {
         for (int j = 0; j < 3; ++j) Hd[i][j] *= (T)M;
       scatter_tet(Hd, B, c, o);
     }
+    return 0.0;
   }
   __device__ double finish(int g, T acc[3]) const {
     double vv[3] = {(double)Vd[g], (double)Vd[(size_t)nV + g], (double)Vd[2 * (size_t)nV + g]};
@@ -2919,10 +2852,10 @@ void launch_local_step(const TileMesh& tm, const RefOp& ro, const double* X, dou
 }
 
 void launch_adj_local32(const TileMesh& tm, const RefOp& ro, const double* X, float* K, double M, double prox,
-                        const SoftDev& sd, float* rhs, float* invd, float* halo, int* n_inverted, hipStream_t st) {
-  const AdjLocalOp32 op{ro, tm.nV, tm.nH, tm.conn, X, K, M, prox, sd, rhs, invd, n_inverted};
-  if (ro.mode == REF_CUBE) launch_scatter<float, 6>(tm, AdjLocalCubeOp32{op}, halo, nullptr, nullptr, st);
-  else launch_scatter<float, 6>(tm, op, halo, nullptr, nullptr, st);
+                        const SoftDev& sd, float* rhs, float* invd, float* halo, double* hex_part, int* n_inverted,
+                        hipStream_t st) {
+  AdjLocalOp32 op{ro, tm.nV, tm.nH, tm.conn, X, K, M, prox, sd, rhs, invd, n_inverted};
+  launch_scatter<float, 6>(tm, op, halo, nullptr, nullptr, st, hex_part);
   if (sd.nL > 0)
     hipLaunchKernelGGL(line_rhs32_kernel, dim3((sd.nL + 255) / 256), dim3(256), 0, st, sd, tm.nV, X,
                        rhs + 3 * (size_t)tm.nV, invd + 3 * (size_t)tm.nV);

@@ -26,7 +26,7 @@ def weight2(s):
 
 
 @pytest.mark.parametrize("cube", [True, False])
-@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("precision", [64])
 def test_weights_rhs_and_diagonal(cube, precision):
     from pyhexopt import capi, meshgen as mg
     rng = np.random.default_rng(11)
