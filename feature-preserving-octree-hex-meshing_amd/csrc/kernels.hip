@@ -1887,7 +1887,7 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
 // current positions and a_L = 0). Before, an iteration took seven launches and moved the
 // direction, the product and the residual through HBM between them: operator tiles 170 us, halo
 // fold 34, line rows 5, alpha 8, vector update 48, beta 5, direction 18 = 288 us at 1.1M hexes;
-// now 165 us for the operator pass and 78 us for the vector pass.
+// now 157 us for the operator pass and 78 us for the vector pass.
 
 // The operator pass. Persistent blocks, the tiles of an XCD dealt as in cg32_apply_pipe_kernel.
 // A hex's 48 FP64 operator values alone would fill 96 registers, so nothing is held for a tile
@@ -2378,7 +2378,7 @@ __device__ __forceinline__ double first_step(double tmin) {
 // line search's first step, which follows from *tmin (part1). They go in one launch, with the step
 // formed here, because a search almost always ends at its first step: the host then reads bound
 // and energies once instead of twice and three launches go. One FP64 iteration on 729 hexes
-// 745 -> 648 us, with the other read-backs joined too. (Both energies in one thread needs 344
+// 745 -> 632 us, with the other read-backs joined too. (Both energies in one thread needs 344
 // registers instead of 124, and 1.1M hexes then lose 150 us.)
 template <class T, bool DIFF, class DT>
 __global__ __launch_bounds__(256) void energy_kernel(RefOp ro, const double* cur, const DT* dst, double step, int nV, const int* conn,
