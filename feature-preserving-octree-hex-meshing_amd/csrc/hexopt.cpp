@@ -69,7 +69,7 @@ struct hexopt_ctx {
   DevBuf d_invs, d_B, d_hflag;
   int ref_mode = -1;
   // SLIM state
-  DevBuf d_K, d_rhs, d_invd, d_x, d_r, d_z, d_p, d_p2, d_tmp, d_halo, d_part[8];
+  DevBuf d_K, d_rhs, d_invd, d_x, d_r, d_z, d_p, d_tmp, d_halo, d_part[8];
   // what the host reads back, in one device block and one pinned copy of it, so that a line search
   // takes one transfer: 16 scalars, the CG state, the state of the last direction solve, counters
   DevBuf d_scal;
@@ -199,11 +199,9 @@ int ensure_state(hexopt_ctx* c) {
   const int nV = c->L.nV, nH = c->L.nH;
   const size_t n = (size_t)3 * nV + c->nL;
   HIPCHK(c, c->d_K.ensure((size_t)48 * nH * sizeof(double)));
-  for (DevBuf* b : {&c->d_rhs, &c->d_invd, &c->d_x, &c->d_r, &c->d_z, &c->d_p, &c->d_p2, &c->d_tmp})
+  for (DevBuf* b : {&c->d_rhs, &c->d_invd, &c->d_x, &c->d_r, &c->d_z, &c->d_p, &c->d_tmp})
     HIPCHK(c, b->ensure(n * sizeof(double)));
-  // 6 values per halo slot in the local step, 3 per (tile, vertex) pair in the CG
-  HIPCHK(c, c->d_halo.ensure(std::max((size_t)6 * (c->L.nSlots + 1), (size_t)3 * (c->L.lv_gid.size() + 1)) *
-                             sizeof(double)));
+  HIPCHK(c, c->d_halo.ensure((size_t)6 * (c->L.nSlots + 1) * sizeof(double)));
   const size_t np = (size_t)std::max(std::max(std::max(c->L.nTiles, nblocks(n)), (nH + 255) / 256 + 1),
                                      std::max(2048, (nV + c->nL + 255) / 256 + 1)) + 64;
   const size_t npf = (size_t)(c->L.nShared + 255) / 256 + 1;
@@ -216,13 +214,6 @@ SoftDev soft_with(hexopt_ctx* c, const hexopt_params* prm);
 
 // per-tet M: weight_opt unless the caller gives tet_mass (the igl::slim variant's weight_opt / 2)
 double tet_mass(const hexopt_params* prm) { return prm->tet_mass > 0 ? prm->tet_mass : prm->weight_opt; }
-
-Cg64 cg64_buffers(hexopt_ctx* c) {
-  Cg64 w{c->d_x.as<double>(), c->d_r.as<double>(), c->d_z.as<double>(), {c->d_p.as<double>(), c->d_p2.as<double>()},
-         c->d_tmp.as<double>(), c->d_halo.as<double>(), cg_state(c), {}};
-  for (int i = 0; i < 8; ++i) w.part[i] = c->d_part[i].as<double>();
-  return w;
-}
 
 struct EnergyParts {
   double* p[4];
@@ -321,8 +312,7 @@ hexopt_ctx* hexopt_create(int nV, const double* V, int nH, const int32_t* hexes,
                    c->d_tile_col.as<uint16_t>(), c->d_tile_lv.as<int>(), c->d_lv_gid.as<int>(),
                    c->d_lv_slot.as<int>(), c->d_lidx.as<uint16_t>(),
                    c->d_sv_gid.as<int>(), c->d_sv_off.as<int>(), c->d_sv_slots.as<int>(),
-                   c->d_tile_corner.as<uint8_t>(), c->d_lv_pair.as<int>(), c->d_v_dst.as<int>(),
-                   (int)L.lv_gid.size()};
+                   c->d_tile_corner.as<uint8_t>(), c->d_lv_pair.as<int>(), c->d_v_dst.as<int>()};
   hexopt_constraints none{};
   if (hexopt_set_constraints(c, &none) != HEXOPT_OK) {
     g_create_error = c->err;
@@ -603,21 +593,17 @@ int hexopt_slim_solve(hexopt_ctx* c, const hexopt_params* prm, int iters, hexopt
                                hipMemcpyDeviceToDevice, st));
       HIPCHK(c, hipMemcpyAsync(c->d_invd.as<double>() + 3 * (size_t)nV, c->d_invd_a.p, nL * sizeof(double),
                                hipMemcpyDeviceToDevice, st));
+      HIPCHK(c, hipMemsetAsync(x + 3 * (size_t)nV, 0, nL * sizeof(double), st));
     }
-    if (!c->glue) {
-      // CG warm start at the current positions (a_L guess 0)
-      const Cg64 w = cg64_buffers(c);
-      launch_cg64(c->tm, ro, c->d_K.as<double>(), prox, sd, c->d_iso.as<int>(), c->n_iso, cur, c->d_rhs.as<double>(),
-                  c->d_invd.as<double>(), w, 20, 1e-8, st);
-    } else {
+    double* pt = c->d_part[2].as<double>();
+    double* pf = c->d_part[3].as<double>();
+    double* pl2 = c->d_part[4].as<double>();
+    const int nfix = (c->L.nShared + 255) / 256, nline = (nL + 255) / 256;
+    double* gsum = c->glue ? c->d_gsum.as<double>() : nullptr;
+    if (c->glue) {
       // known_value_post (slim_m.cpp:403-475): the pinned rows leave the system. Its right-hand
       // side is rhs - L x_pinned on the free rows, and the CG runs on the free rows from the
       // free part of the current positions (pinned rows of r, z and p stay 0)
-      double* pt = c->d_part[2].as<double>();
-      double* pf = c->d_part[3].as<double>();
-      double* pl2 = c->d_part[4].as<double>();
-      const int nfix = (c->L.nShared + 255) / 256;
-      double* gsum = c->d_gsum.as<double>();
       double* xfix = c->d_xfix.as<double>();
       launch_glue_split(nV, c->d_invd.as<double>(), cur, xfix, x, st);
       launch_group_sum(sd, nV, xfix, gsum, st);
@@ -625,20 +611,23 @@ int hexopt_slim_solve(hexopt_ctx* c, const hexopt_params* prm, int iters, hexopt
                    pf, pl2, st);
       launch_glue_rhs(nV, c->d_invd.as<double>(), c->d_rhs.as<double>(), c->d_tmp.as<double>(), st);
       launch_group_sum(sd, nV, x, gsum, st);
-      launch_apply(c->tm, ro, c->d_K.as<double>(), x, c->d_tmp.as<double>(), prox, sd, c->d_halo.as<double>(), pt, pf,
-                   pl2, st);
-      launch_cg_init(n, c->d_rhs.as<double>(), c->d_tmp.as<double>(), c->d_r.as<double>(), c->d_part[0].as<double>(),
-                     c->d_part[1].as<double>(), nb, cg_state(c), c->d_invd.as<double>(), c->d_p.as<double>(),
-                     c->d_part[5].as<double>(), 1e-8, st);
-      for (int k = 0; k < 20; ++k) {
-        launch_group_sum(sd, nV, c->d_p.as<double>(), gsum, st);
-        launch_apply(c->tm, ro, c->d_K.as<double>(), c->d_p.as<double>(), c->d_tmp.as<double>(), prox, sd,
-                     c->d_halo.as<double>(), pt, pf, pl2, st);
-        launch_cg_alpha(cg_state(c), pt, c->L.nTiles, pf, nfix, pl2, 0, st);
-        launch_cg_update(n, cg_state(c), x, c->d_r.as<double>(), c->d_z.as<double>(), c->d_p.as<double>(),
-                         c->d_tmp.as<double>(), c->d_invd.as<double>(), c->d_part[6].as<double>(),
-                         c->d_part[7].as<double>(), nb, c->d_p.as<double>(), st);
-      }
+    } else {
+      // CG warm start at the current positions (a_L guess 0)
+      HIPCHK(c, hipMemcpyAsync(x, cur, 3 * (size_t)nV * sizeof(double), hipMemcpyDeviceToDevice, st));
+    }
+    launch_apply(c->tm, ro, c->d_K.as<double>(), x, c->d_tmp.as<double>(), prox, sd, c->d_halo.as<double>(), pt, pf,
+                 pl2, st);
+    launch_cg_init(n, c->d_rhs.as<double>(), c->d_tmp.as<double>(), c->d_r.as<double>(), c->d_part[0].as<double>(),
+                   c->d_part[1].as<double>(), nb, cg_state(c), c->d_invd.as<double>(), c->d_p.as<double>(),
+                   c->d_part[5].as<double>(), 1e-8, st);
+    for (int k = 0; k < 20; ++k) {
+      if (c->glue) launch_group_sum(sd, nV, c->d_p.as<double>(), gsum, st);
+      launch_apply(c->tm, ro, c->d_K.as<double>(), c->d_p.as<double>(), c->d_tmp.as<double>(), prox, sd,
+                   c->d_halo.as<double>(), pt, pf, pl2, st);
+      launch_cg_alpha(cg_state(c), pt, c->L.nTiles, pf, nfix, pl2, nline, st);
+      launch_cg_update(n, cg_state(c), x, c->d_r.as<double>(), c->d_z.as<double>(), c->d_p.as<double>(),
+                       c->d_tmp.as<double>(), c->d_invd.as<double>(), c->d_part[6].as<double>(),
+                       c->d_part[7].as<double>(), nb, c->d_p.as<double>(), st);
     }
     launch_cg_zero_if(n, cg_state(c), x, nb, st);
     if (c->glue) launch_glue_restore(nV, c->d_invd.as<double>(), cur, x, st);
@@ -1091,7 +1080,8 @@ int hexopt_time_kernel(hexopt_ctx* c, int which, int reps, double* ms_per_launch
   auto one = [&]() {
     switch (which) {
       case 0:
-        launch_cg64_operator(tm, ro, c->d_K.as<double>(), sd, c->d_cur.as<double>(), cg64_buffers(c), st);
+        launch_apply(tm, ro, c->d_K.as<double>(), c->d_p.as<double>(), c->d_tmp.as<double>(), 1e-5, sd,
+                     c->d_halo.as<double>(), c->d_part[2].as<double>(), nullptr, nullptr, st);
         break;
       case 1:
         // as inside the CG loop after its first iteration: the previous beta step formed from

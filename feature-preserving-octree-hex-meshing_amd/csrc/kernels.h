@@ -22,7 +22,6 @@ struct TileMesh {
   const uint8_t* tile_corner;
   const int* lv_pair; // per local vertex: id (top bit: first tile) and place among all (tile, vertex) pairs
   const int* v_dst;   // nV+1: each vertex's run of places
-  int nPairs;         // number of those pairs
 };
 
 enum RefMode { REF_CUBE = 0, REF_GENERAL = 1 };
@@ -149,20 +148,6 @@ void launch_cg32_iteration(const TileMesh& tm, const RefOp& ro, const float* K, 
                            float* out, float* halo, const float* invd, float* x, float* r, float* zout, void* state,
                            double* part_tile, double* part_rr, double* part_rz, double* part_qz, double* part_bzq,
                            double* part_qq, int k, int last, hipStream_t st);
-// FP64 CG (Eigen's algorithm with its Jacobi preconditioner) on L x = rhs from x = cur, a_L = 0:
-// the solution goes to x, both vectors with 3 nV + nL entries. out: the a_L rows of the product;
-// halo: 3 * nPairs values; part: 8 arrays of partials; sd without glue.
-struct Cg64 {
-  double *x, *r, *z, *p[2], *out, *halo;
-  void* state;
-  double* part[8];
-};
-void launch_cg64(const TileMesh& tm, const RefOp& ro, const double* K, double prox, const SoftDev& sd, const int* iso,
-                 int niso, const double* cur, const double* rhs, const double* invd, const Cg64& w, int iters,
-                 double tol, hipStream_t st);
-// its operator pass alone (the one that forms the first residual)
-void launch_cg64_operator(const TileMesh& tm, const RefOp& ro, const double* K, const SoftDev& sd, const double* cur,
-                          const Cg64& w, hipStream_t st);
 void launch_f2d(int n, const float* a, double* b, hipStream_t st);
 void launch_d2f(int n, const double* a, float* b, hipStream_t st);
 // b = -g / 2 on the vertex rows of g (the FP64 adjoint gradient, in place) and the a_L rows at

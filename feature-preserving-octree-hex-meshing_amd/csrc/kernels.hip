@@ -1308,7 +1308,7 @@ __global__ void cg_zero_if_kernel(int n, const CGState* st, T* x) {
 //                alpha = r.z / (p.E p + p.R p). p.R p needs no pass of its own: with
 //                p = z + beta q (q the previous direction) it is
 //                z.R z + 2 beta z.R q + beta^2 q.R q, three sums the previous update left
-//   cg_vertex    per vertex: E p (its tile's value or the sum of its halo slots) + R p,
+//   cg32_update  per vertex: E p (its tile's value or the sum of its halo slots) + R p,
 //                x += alpha p, r -= alpha L p, z = r / diag for the vertex and its line
 //                unknown; FP64 partials of |r|^2, r.z and of z.R z, z.R p, p.R p
 //   cg32_beta    one block: convergence test, beta, and the three R sums
@@ -1505,13 +1505,12 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_kernel(TileMesh tm, RefOp
 }
 
 // line unknown i: p_a = z_a + beta p_prev_a and the a_L row (L p)_a = lamL (|t|^2 p_a - t.p_v)
-template <class T>
-__device__ __forceinline__ void line_row(const SoftDev& sd, int nV, const T* __restrict__ z,
-                                         const T* __restrict__ pprev, T* __restrict__ pnew, T* __restrict__ out,
-                                         T beta, int i) {
+__device__ __forceinline__ void line_row(const SoftDev& sd, int nV, const float* __restrict__ z,
+                                         const float* __restrict__ pprev, float* __restrict__ pnew,
+                                         float* __restrict__ out, float beta, int i) {
   const size_t nA = 3 * (size_t)nV;
   const int v = sd.lv[i];
-  const T pa = z[nA + i] + beta * pprev[nA + i];
+  const float pa = z[nA + i] + beta * pprev[nA + i];
   pnew[nA + i] = pa;
   const double* t = sd.lt + (size_t)i * 3;
   double tp = 0, tt = 0;
@@ -1521,7 +1520,7 @@ __device__ __forceinline__ void line_row(const SoftDev& sd, int nV, const T* __r
     tp += t[d] * pv;
     tt += t[d] * t[d];
   }
-  out[nA + i] = (T)(sd.lamL * (tt * (double)pa - tp));
+  out[nA + i] = (float)(sd.lamL * (tt * (double)pa - tp));
 }
 
 // The beta step of CG iteration up.k (cg32_beta_kernel's), formed by every block of the next
@@ -1770,24 +1769,14 @@ __global__ __launch_bounds__(256) void cg32_lines_kernel(SoftDev sd, int nV, con
 // each line unknown belongs to exactly one vertex). With ntiles > 0 every block first forms
 // alpha itself from the operator pass's ntiles partials, as cg32_alpha_kernel would (the
 // same sum in every block, so every block holds the same alpha).
-// E p: float, a float4 per place; double, three planes of tm.nPairs places.
-__device__ __forceinline__ void add_place(const float* halo, int nP, int k, double a[3]) {
-  const float4 h = reinterpret_cast<const float4*>(halo)[k];
-  a[0] += (double)h.x; a[1] += (double)h.y; a[2] += (double)h.z;
-}
-__device__ __forceinline__ void add_place(const double* halo, int nP, int k, double a[3]) {
-#pragma unroll
-  for (int d = 0; d < 3; ++d) a[d] += halo[(size_t)d * nP + k];
-}
-
-template <class T>
-__global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd, double prox,
-                                                        const T* __restrict__ halo, const T* __restrict__ p,
-                                                        const T* __restrict__ out, const T* __restrict__ invd,
-                                                        T* __restrict__ x, T* __restrict__ r, T* __restrict__ z,
-                                                        const CGState* st, const double* part_tile, int ntiles,
-                                                        double* part_rr, double* part_rz, double* part_qz,
-                                                        double* part_bzq, double* part_qq) {
+__global__ __launch_bounds__(256) void cg32_update_kernel(TileMesh tm, SoftDev sd, double prox,
+                                                          const float4* __restrict__ halo,
+                                                          const float* __restrict__ p, const float* __restrict__ out,
+                                                          const float* __restrict__ invd, float* __restrict__ x,
+                                                          float* __restrict__ r, float* __restrict__ z,
+                                                          const CGState* st, const double* part_tile, int ntiles,
+                                                          double* part_rr, double* part_rz,
+                                                          double* part_qz, double* part_bzq, double* part_qq) {
   __shared__ double red[5 * 16];
   const int done = st->done;
   const int nV = tm.nV;
@@ -1796,7 +1785,7 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
   // p, r, x, 1/diag and constraint row. The first vertex's go out before alpha is formed, whose
   // partials take as long to come
   int k0, k1;
-  T pf[3], rf[3], xf[3], df[3];
+  float pf[3], rf[3], xf[3], df[3];
   int2 cl;
   auto load = [&](int g) {
     k0 = tm.v_dst[g];
@@ -1813,18 +1802,18 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
   };
   int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g < nV) load(g);
-  T alpha;
+  float alpha;
   if (ntiles > 0) {
     const double* const pt[1] = {part_tile};
     double ev[1];
     sum_parts_n_wide<1, 4>(pt, ntiles, red, ev);
     if (done) return;
     const double e = ev[0];
-    const double b = (double)(T)st->beta;
-    alpha = (T)(st->absNew / (e + st->qz + 2.0 * b * st->bzq + b * b * st->qq));
+    const double b = (double)(float)st->beta;
+    alpha = (float)(st->absNew / (e + st->qz + 2.0 * b * st->bzq + b * b * st->qq));
   } else {
     if (done) return;
-    alpha = (T)st->alpha;
+    alpha = (float)st->alpha;
   }
   double srr = 0, srz = 0, fz = 0, fzq = 0, fq = 0;
   for (bool first = true; g < nV; g += gridDim.x * blockDim.x, first = false) {
@@ -1838,20 +1827,23 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
     const double pa = ln >= 0 ? (double)p[nA + ln] : 0.0;
     double vr[3];
     vertex_rows(sd, prox, ci, ln, pv, pa, vr);
-    double a[3] = {0.0, 0.0, 0.0}, a1[3] = {0.0, 0.0, 0.0};
-    if (k1 > k0) add_place(halo, tm.nPairs, k0, a);
-    if (k1 > k0 + 1) add_place(halo, tm.nPairs, k0 + 1, a1);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) a[d] += a1[d];
-    for (int k = k0 + 2; k < k1; ++k) add_place(halo, tm.nPairs, k, a);
+    const float4 h0 = k1 > k0 ? halo[k0] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 h1 = k1 > k0 + 1 ? halo[k0 + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
+    double a[3] = {0.0, 0.0, 0.0};
+    if (k1 > k0) { a[0] += (double)h0.x; a[1] += (double)h0.y; a[2] += (double)h0.z; }
+    if (k1 > k0 + 1) { a[0] += (double)h1.x; a[1] += (double)h1.y; a[2] += (double)h1.z; }
+    for (int k = k0 + 2; k < k1; ++k) {
+      const float4 hv = halo[k];
+      a[0] += (double)hv.x; a[1] += (double)hv.y; a[2] += (double)hv.z;
+    }
     double zn[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       const size_t j = (size_t)d * nV + g;
       x[j] = xf[d] + alpha * pf[d];
-      const T rv = rf[d] - alpha * (T)(a[d] + vr[d]);
+      const float rv = rf[d] - alpha * (float)(a[d] + vr[d]);
       r[j] = rv;
-      const T zv = df[d] * rv;
+      const float zv = df[d] * rv;
       z[j] = zv;
       zn[d] = (double)zv;
       srr += (double)rv * (double)rv;
@@ -1861,9 +1853,9 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
     if (ln >= 0) {
       const size_t j = nA + ln;
       x[j] += alpha * p[j];
-      const T rv = r[j] - alpha * out[j];
+      const float rv = r[j] - alpha * out[j];
       r[j] = rv;
-      const T zv = invd[j] * rv;
+      const float zv = invd[j] * rv;
       z[j] = zv;
       za = (double)zv;
       srr += (double)rv * (double)rv;
@@ -1879,261 +1871,6 @@ __global__ __launch_bounds__(256) void cg_vertex_kernel(TileMesh tm, SoftDev sd,
   if (threadIdx.x == 0) {
     part_rr[blockIdx.x] = v[0]; part_rz[blockIdx.x] = v[1];
     part_qz[blockIdx.x] = v[2]; part_bzq[blockIdx.x] = v[3]; part_qq[blockIdx.x] = v[4];
-  }
-}
-
-// ---------------------------------------------------------------------------------------
-// FP64 CG of the plain path in the same two passes (the position form: L x = rhs from x = the
-// current positions and a_L = 0). Before, an iteration took seven launches and moved the
-// direction, the product and the residual through HBM between them: operator tiles 170 us, halo
-// fold 34, line rows 5, alpha 8, vector update 48, beta 5, direction 18 = 288 us at 1.1M hexes;
-// now 157 us for the operator pass and 78 us for the vector pass.
-
-// The operator pass. Persistent blocks, the tiles of an XCD dealt as in cg32_apply_pipe_kernel.
-// A hex's 48 FP64 operator values alone would fill 96 registers, so nothing is held for a tile
-// ahead: the corner values stay in LDS and are read again by every tet, the operator values come
-// pair by pair, and the registers this leaves free let three blocks share a CU and cover each
-// other's loads. (With the next tile's ids, z and p fetched ahead, 30 to 90 registers spill.)
-// What a block waits for before its first tile is a chain of loads, and on a mesh of a few tiles
-// that chain is the pass: so the first tile's z and previous direction go to LDS, where they need
-// no registers, while the partials of beta are on their way, and are combined once beta is known.
-// Per call, loads after beta and as here: 150 -> 144 us on 1.1M hexes, 35.4 -> 33.3 us on 262,144,
-// 8.8 -> 7.7 us on 729.
-// START: the pass that forms E x for the first residual (z = the positions, no direction before
-// it, a_L = 0).
-template <bool CUBE, bool START>
-__global__ __launch_bounds__(kTileHex, CUBE ? 3 : 2) void cg64_apply_kernel(TileMesh tm, RefOp ro, const double* __restrict__ K,
-                                                                 const double* __restrict__ z,
-                                                                 const double* __restrict__ pprev,
-                                                                 double* __restrict__ pnew, double* __restrict__ out,
-                                                                 double* __restrict__ halo, SoftDev sd,
-                                                                 const int* __restrict__ iso, int niso, CGState* st,
-                                                                 double* partial, UpdParts up) {
-  __shared__ double sp[3 * kMaxLV];
-  __shared__ double acc[3 * kMaxLV];
-  __shared__ double red[5 * 16];
-  const int tid = threadIdx.x;
-  const int nV = tm.nV, nH = tm.nH, nT = tm.nTiles;
-  const size_t nA = 3 * (size_t)nV;
-  const int q8 = nT / 8, r8 = nT % 8;
-  const int x = blockIdx.x % 8, rank = blockIdx.x / 8;
-  const int nb = ((int)gridDim.x + 7 - x) / 8;  // blocks on XCD x
-  const int tend = (x + 1) * q8 + (x + 1 < r8 ? x + 1 : r8);
-  int tile = x * q8 + (x < r8 ? x : r8) + rank;
-  int h0 = 0, nh = 0, lv0 = 0, nlv = 0, corner = 0;
-  auto head = [&]() {
-    h0 = tm.tile_hex[tile];
-    nh = tm.tile_hex[tile + 1] - h0;
-    lv0 = tm.tile_lv[tile];
-    nlv = tm.tile_lv[tile + 1] - lv0;
-    corner = tm.tile_corner[tile];
-  };
-  double beta = 0.0;
-  bool raw = false;  // the tile's z is in sp and its previous direction in acc
-  if constexpr (START) {
-    if (tile < tend) head();
-  } else {
-    const int done = st->done;
-    BetaParts bp;
-    if (up.n > 0) load_beta(up, bp);
-    if (tile < tend) {
-      head();
-      for (int lv = tid; lv < nlv; lv += kTileHex) {
-        const int g = tm.lv_pair[2 * (size_t)(lv0 + lv)] & 0x7fffffff;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const size_t j = (size_t)d * nV + g;
-          sp[d * kMaxLV + lv] = z[j];
-          acc[d * kMaxLV + lv] = pprev[j];
-        }
-      }
-      raw = true;
-    }
-    if (up.n > 0) {
-      if (form_beta(st, up, bp, done, red, beta)) return;
-    } else if (done) {
-      return;
-    }
-  }
-  // the work outside the tiles: line unknowns, and p of the vertices without hexes
-  for (int i = blockIdx.x * kTileHex + tid; i < sd.nL; i += gridDim.x * kTileHex) {
-    if constexpr (START) {
-      const int v = sd.lv[i];
-      const double* t = sd.lt + (size_t)i * 3;
-      double tp = 0;
-#pragma unroll
-      for (int d = 0; d < 3; ++d) tp += t[d] * z[(size_t)d * nV + v];
-      pnew[nA + i] = 0.0;
-      out[nA + i] = -sd.lamL * tp;
-    } else {
-      line_row<double>(sd, nV, z, pprev, pnew, out, beta, i);
-    }
-  }
-  for (int i = blockIdx.x * kTileHex + tid; i < niso; i += gridDim.x * kTileHex) {
-    const int g = iso[i];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const size_t j = (size_t)d * nV + g;
-      pnew[j] = START ? z[j] : z[j] + beta * pprev[j];
-    }
-  }
-  double part = 0.0;
-  while (tile < tend) {
-    const bool active = tid < nh;
-    int li[8];
-    double kp[2][12];
-    if (active) {
-      load_li(tm, h0 + tid, li);
-      if constexpr (CUBE) k_pair(K, nH, h0 + tid, 0, kp[0]);
-    }
-    for (int lv = tid; lv < nlv; lv += kTileHex) {
-      const int2 pair = reinterpret_cast<const int2*>(tm.lv_pair)[lv0 + lv];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const size_t j = (size_t)d * nV + (pair.x & 0x7fffffff);
-        const double pv = START ? z[j] : raw ? sp[d * kMaxLV + lv] + beta * acc[d * kMaxLV + lv] : z[j] + beta * pprev[j];
-        sp[d * kMaxLV + lv] = pv;
-        acc[d * kMaxLV + lv] = 0.0;
-        if (pair.x < 0) pnew[j] = pv;
-      }
-    }
-    __syncthreads();
-    double c[8][3];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) c[k][d] = 0.0;
-    if (active) {
-      if constexpr (CUBE) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          // the next pair's values are on their way while this pair's tets run; the barrier keeps
-          // the scheduler from fetching all four pairs at once
-          if ((t & 1) == 0) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (t < 6) k_pair(K, nH, h0 + tid, t / 2 + 1, kp[(t / 2 + 1) & 1]);
-          }
-          const double* kk = kp[(t / 2) & 1] + 6 * (t & 1);
-          double E[3][3];
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            const double o = sp[d * kMaxLV + li[kHexTet[t][0]]];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) E[d][k] = sp[d * kMaxLV + li[kHexTet[t][k + 1]]] - o;
-          }
-#pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            const double f0 = kk[0] * E[0][k] + kk[3] * E[1][k] + kk[4] * E[2][k];
-            const double f1 = kk[3] * E[0][k] + kk[1] * E[1][k] + kk[5] * E[2][k];
-            const double f2 = kk[4] * E[0][k] + kk[5] * E[1][k] + kk[2] * E[2][k];
-            const int vk = kHexTet[t][k + 1], v0 = kHexTet[t][0];
-            c[vk][0] += f0; c[vk][1] += f1; c[vk][2] += f2;
-            c[v0][0] -= f0; c[v0][1] -= f1; c[v0][2] -= f2;
-            part += E[0][k] * f0 + E[1][k] * f1 + E[2][k] * f2;
-          }
-        }
-      } else {
-        double q[8][3];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-#pragma unroll
-          for (int d = 0; d < 3; ++d) q[k][d] = sp[d * kMaxLV + li[k]];
-        hex_forces<double, double>(ro, K, nH, h0 + tid, q, c);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-#pragma unroll
-          for (int d = 0; d < 3; ++d) part += sp[d * kMaxLV + li[k]] * c[k][d];
-      }
-    }
-    scatter_tile<double, 3>(tm, tile, corner, nh, active, li, c, acc);
-    for (int lv = tid; lv < nlv; lv += kTileHex) {
-      const int k = tm.lv_pair[2 * (size_t)(lv0 + lv) + 1];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) halo[(size_t)d * tm.nPairs + k] = acc[d * kMaxLV + lv];
-    }
-    tile += nb;
-    if (tile < tend) head();
-    raw = false;
-    __syncthreads();  // the next tile's staging overwrites sp and acc
-  }
-  const double bs = block_sum(part, red);
-  if (tid == 0) partial[blockIdx.x] = bs;
-}
-
-// The first residual r = rhs - L x of x = p (written by the start pass), z = r / diag, and the
-// partials of |rhs|^2, |r|^2, r.z and z.R z (the first direction is z)
-__global__ __launch_bounds__(256) void cg64_start_kernel(TileMesh tm, SoftDev sd, double prox,
-                                                         const double* __restrict__ halo, const double* __restrict__ p,
-                                                         const double* __restrict__ out, const double* __restrict__ rhs,
-                                                         const double* __restrict__ invd, double* __restrict__ x,
-                                                         double* __restrict__ r, double* __restrict__ z, double* part_b,
-                                                         double* part_rr, double* part_rz, double* part_qz) {
-  __shared__ double red[4 * 16];
-  const int nV = tm.nV;
-  const size_t nA = 3 * (size_t)nV;
-  double sb = 0, srr = 0, srz = 0, fz = 0;
-  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < nV; g += gridDim.x * blockDim.x) {
-    const int2 cl = sd.cl ? reinterpret_cast<const int2*>(sd.cl)[g] : make_int2(-1, -1);
-    const int ci = cl.x, ln = cl.y;
-    double pv[3], vr[3], a[3] = {0.0, 0.0, 0.0}, zn[3], za = 0.0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) pv[d] = p[(size_t)d * nV + g];
-    vertex_rows(sd, prox, ci, ln, pv, 0.0, vr);
-    for (int k = tm.v_dst[g]; k < tm.v_dst[g + 1]; ++k) add_place(halo, tm.nPairs, k, a);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const size_t j = (size_t)d * nV + g;
-      const double b = rhs[j], rv = b - (a[d] + vr[d]);
-      x[j] = pv[d];
-      r[j] = rv;
-      z[j] = zn[d] = invd[j] * rv;
-      sb += b * b;
-      srr += rv * rv;
-      srz += rv * zn[d];
-    }
-    if (ln >= 0) {
-      const size_t j = nA + ln;
-      const double b = rhs[j], rv = b - out[j];
-      x[j] = 0.0;
-      r[j] = rv;
-      z[j] = za = invd[j] * rv;
-      sb += b * b;
-      srr += rv * rv;
-      srz += rv * za;
-    }
-    fz += vertex_form(sd, prox, ci, ln, zn, za, zn, za);
-  }
-  double v[4] = {sb, srr, srz, fz};
-  block_sum_n<4>(v, red);
-  if (threadIdx.x == 0) {
-    part_b[blockIdx.x] = v[0]; part_rr[blockIdx.x] = v[1];
-    part_rz[blockIdx.x] = v[2]; part_qz[blockIdx.x] = v[3];
-  }
-}
-
-// ConjugateGradient.h:44-62
-__global__ void cg64_start_fin_kernel(CGState* st, const double* part_b, const double* part_rr, const double* part_rz,
-                                      const double* part_qz, int nb, double tol) {
-  __shared__ double red[4 * 16];
-  const double* const parts[4] = {part_b, part_rr, part_rz, part_qz};
-  double v[4];
-  sum_parts_n<4>(parts, nb, red, v);
-  if (threadIdx.x == 0) {
-    st->rhsNorm2 = v[0];
-    st->iters = 0;
-    st->done = 0;
-    st->zero_rhs = 0;
-    st->beta = 0;
-    st->qz = v[3];
-    st->bzq = 0;
-    st->qq = 0;
-    if (v[0] == 0) { st->done = 1; st->zero_rhs = 1; st->tol_error = 0; return; }
-    st->threshold = tol * tol * v[0];
-    st->rn2 = v[1];
-    if (v[1] < st->threshold) { st->done = 1; st->tol_error = sqrt(v[1] / v[0]); return; }
-    st->absNew = v[2];
-    st->hist[0] = v[2];
-    st->hist[1] = 0;
   }
 }
 
@@ -3013,7 +2750,6 @@ int launch_cg32_apply(const TileMesh& tm, const RefOp& ro, const float* K, const
 // blocks of the grid-stride update pass: as many as are resident at once on the device (so
 // no block waits for another to finish all its vertices), which keeps the following one-block
 // reduction of their partials short
-template <class T>
 static int update_grid(int nV) {
   static int fit[64] = {0};
   int dev = 0;
@@ -3022,7 +2758,7 @@ static int update_grid(int nV) {
   if (dev < 0 || dev >= 64) return std::min(want, 1024);
   if (fit[dev] == 0) {
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cg_vertex_kernel<T>, 256, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cg32_update_kernel, 256, 0) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       per_cu = cus = 0;
     fit[dev] = std::max(64, per_cu * cus);
@@ -3035,7 +2771,7 @@ int launch_cg32_apply_folded(const TileMesh& tm, const RefOp& ro, const float* K
                              void* state, double* part, const double* part_rr, const double* part_rz,
                              const double* part_qz, const double* part_bzq, const double* part_qq, int k,
                              hipStream_t st) {
-  UpdParts up{{part_rr, part_rz, part_qz, part_bzq, part_qq}, update_grid<float>(tm.nV), k};
+  UpdParts up{{part_rr, part_rz, part_qz, part_bzq, part_qq}, update_grid(tm.nV), k};
   return launch_cg32_apply(tm, ro, K, sd, iso, niso, z, pprev, pnew, out, halo, state, part, st, &up);
 }
 
@@ -3048,7 +2784,7 @@ void launch_cg32_iteration(const TileMesh& tm, const RefOp& ro, const float* K, 
   // the operator pass of cube references forms the previous iteration's beta step itself; the
   // one-block beta pass then runs only after the last update
   const bool fold_beta = ro.mode == REF_CUBE;
-  UpdParts up{{part_rr, part_rz, part_qz, part_bzq, part_qq}, update_grid<float>(tm.nV), k - 1};
+  UpdParts up{{part_rr, part_rz, part_qz, part_bzq, part_qq}, update_grid(tm.nV), k - 1};
   // a positive count: the operator pass did the lines and the vertices without hexes
   const int np = launch_cg32_apply(tm, ro, K, sd, iso, niso, z, pprev, pnew, out, halo, cs, part_tile, st,
                                    fold_beta && k > 0 ? &up : nullptr);
@@ -3058,74 +2794,14 @@ void launch_cg32_iteration(const TileMesh& tm, const RefOp& ro, const float* K, 
   if (!fold)
     hipLaunchKernelGGL(cg32_alpha_kernel, dim3(1), dim3(1024), 0, st, cs, (const double*)part_tile, -np, tm.nV, iso,
                        niso, z, pprev, pnew);
-  const int nbu = update_grid<float>(tm.nV);
-  hipLaunchKernelGGL(cg_vertex_kernel<float>, dim3(nbu), dim3(256), 0, st, tm, sd, prox, (const float*)halo,
+  const int nbu = update_grid(tm.nV);
+  hipLaunchKernelGGL(cg32_update_kernel, dim3(nbu), dim3(256), 0, st, tm, sd, prox, (const float4*)halo,
                      (const float*)pnew, (const float*)out, invd, x, r, zout, (const CGState*)cs,
                      (const double*)part_tile, fold ? std::abs(np) : 0, part_rr, part_rz, part_qz, part_bzq, part_qq);
   if (!fold_beta || last)
     hipLaunchKernelGGL(cg32_beta_kernel, dim3(1), dim3(1024), 0, st, cs, (const double*)part_rr,
                        (const double*)part_rz, (const double*)part_qz, (const double*)part_bzq,
                        (const double*)part_qq, nbu);
-}
-
-namespace {
-// blocks of the FP64 operator pass: as many as fit on the device at once
-template <bool CUBE>
-int apply64_grid(int ntiles) {
-  static int fit[64] = {0};
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  if (dev < 0 || dev >= 64) return std::min(ntiles, 8);
-  if (fit[dev] == 0) {
-    int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cg64_apply_kernel<CUBE, false>, kTileHex, 0) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      per_cu = cus = 0;
-    fit[dev] = std::max(8, per_cu * cus);
-  }
-  return std::min(ntiles, fit[dev]);
-}
-
-int cg64_apply(const TileMesh& tm, const RefOp& ro, const double* K, const SoftDev& sd, const int* iso, int niso,
-               const double* z, const double* pprev, double* pnew, const Cg64& w, const UpdParts& up, int start,
-               hipStream_t st) {
-  const bool cube = ro.mode == REF_CUBE;
-  const int grid = std::max(1, cube ? apply64_grid<true>(tm.nTiles) : apply64_grid<false>(tm.nTiles));
-  const auto kernel = cube ? (start ? cg64_apply_kernel<true, true> : cg64_apply_kernel<true, false>)
-                              : (start ? cg64_apply_kernel<false, true> : cg64_apply_kernel<false, false>);
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kTileHex), 0, st, tm, ro, K, z, pprev, pnew, w.out, w.halo, sd, iso, niso,
-                     (CGState*)w.state, w.part[2], up);
-  return grid;
-}
-}  // namespace
-
-void launch_cg64_operator(const TileMesh& tm, const RefOp& ro, const double* K, const SoftDev& sd, const double* cur,
-                          const Cg64& w, hipStream_t st) {
-  (void)cg64_apply(tm, ro, K, sd, nullptr, 0, cur, nullptr, w.p[0], w, UpdParts{}, 1, st);
-}
-
-void launch_cg64(const TileMesh& tm, const RefOp& ro, const double* K, double prox, const SoftDev& sd, const int* iso,
-                 int niso, const double* cur, const double* rhs, const double* invd, const Cg64& w, int iters,
-                 double tol, hipStream_t st) {
-  CGState* cs = (CGState*)w.state;
-  const int nbu = update_grid<double>(tm.nV);
-  (void)cg64_apply(tm, ro, K, sd, iso, niso, cur, nullptr, w.p[0], w, UpdParts{}, 1, st);
-  hipLaunchKernelGGL(cg64_start_kernel, dim3(nbu), dim3(256), 0, st, tm, sd, prox, (const double*)w.halo,
-                     (const double*)w.p[0], (const double*)w.out, rhs, invd, w.x, w.r, w.z, w.part[0], w.part[1],
-                     w.part[4], w.part[5]);
-  hipLaunchKernelGGL(cg64_start_fin_kernel, dim3(1), dim3(1024), 0, st, cs, (const double*)w.part[0],
-                     (const double*)w.part[1], (const double*)w.part[4], (const double*)w.part[5], nbu, tol);
-  for (int k = 0; k < iters; ++k) {
-    UpdParts up{{w.part[4], w.part[5], w.part[3], w.part[6], w.part[7]}, k > 0 ? nbu : 0, k - 1};
-    const int np = cg64_apply(tm, ro, K, sd, iso, niso, w.z, w.p[k & 1], w.p[(k + 1) & 1], w, up, 0, st);
-    hipLaunchKernelGGL(cg_vertex_kernel<double>, dim3(nbu), dim3(256), 0, st, tm, sd, prox, (const double*)w.halo,
-                       (const double*)w.p[(k + 1) & 1], (const double*)w.out, invd, w.x, w.r, w.z, (const CGState*)cs,
-                       (const double*)w.part[2], np, w.part[4], w.part[5], w.part[3], w.part[6], w.part[7]);
-  }
-  if (iters > 0)
-    hipLaunchKernelGGL(cg32_beta_kernel, dim3(1), dim3(1024), 0, st, cs, (const double*)w.part[4],
-                       (const double*)w.part[5], (const double*)w.part[3], (const double*)w.part[6],
-                       (const double*)w.part[7], nbu);
 }
 
 void launch_max_step(const double* cur, const double* dst, int nV, const int* conn, int nH, double* part,

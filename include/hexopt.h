@@ -171,7 +171,7 @@ int hexopt_opt32_solve(hexopt_ctx* ctx, const hexopt_params* prm, const hexopt_o
 int hexopt_debug_operator(hexopt_ctx* ctx, const hexopt_params* prm, int precision, double* K);
 
 /* Average duration (ms, HIP events on the context's stream) of one launch of a kernel:
- * 0 FP64 CG operator pass (cg64_apply, forming the first residual's product), 1 FP32 fused CG operator pass (cg32_apply, forming the previous
+ * 0 FP64 CG operator tile pass, 1 FP32 fused CG operator pass (cg32_apply, forming the previous
  * iteration's beta step as it does inside the CG loop), 2 FP64 local step
  * tile pass, 3 FP32 adjoint/local tile pass, 4 the FP32 energy + gradient pass of
  * hexopt_energy_grad (CURRENT rounded to FP32), 5 the same in FP64. Modes 0-3 need a prior

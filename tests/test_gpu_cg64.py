@@ -1,6 +1,6 @@
-"""The fused FP64 CG against the same 20 steps in numpy on the operator of hexopt_debug_system,
-which is applied by other kernels: one partly filled tile, several tiles, feature lines, a vertex
-without hexes, both reference operators."""
+"""The FP64 CG of slim_solve against the same 20 steps in numpy on the operator of
+hexopt_debug_system: one partly filled tile, several tiles, feature lines, a vertex without hexes,
+both reference operators."""
 import numpy as np
 import pytest
 
