@@ -220,162 +220,6 @@ __device__ void slim_weights(const T J[3][3], int energy, T exp_f, T W[3][3], T 
     }
 }
 
-// Cofactor matrix (det X times the inverse transpose)
-__device__ __forceinline__ void cofactor3(const double X[3][3], double C[3][3]) {
-  C[0][0] = X[1][1] * X[2][2] - X[1][2] * X[2][1]; C[0][1] = X[1][2] * X[2][0] - X[1][0] * X[2][2];
-  C[0][2] = X[1][0] * X[2][1] - X[1][1] * X[2][0]; C[1][0] = X[0][2] * X[2][1] - X[0][1] * X[2][2];
-  C[1][1] = X[0][0] * X[2][2] - X[0][2] * X[2][0]; C[1][2] = X[0][1] * X[2][0] - X[0][0] * X[2][1];
-  C[2][0] = X[0][1] * X[1][2] - X[0][2] * X[1][1]; C[2][1] = X[0][2] * X[1][0] - X[0][0] * X[1][2];
-  C[2][2] = X[0][0] * X[1][1] - X[0][1] * X[1][0];
-}
-
-__device__ __forceinline__ double norm2_3(const double X[3][3]) {
-  double s = 0.0;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) s += X[i][j] * X[i][j];
-  return s;
-}
-
-// 1 / x to within an ulp or so: the hardware's approximation (good to about 2^-25) and two
-// Newton steps. Only for values well inside the normal range.
-__device__ __forceinline__ double fast_rcp(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = r + r * (1.0 - x * r);
-  return r + r * (1.0 - x * r);
-}
-
-// One scaled step of sd_polar's iteration, Q = (g X + X^-T / g) / 2 from X, its cofactors C and
-// det X; any positive weights of the two terms keep the polar factor, so the scale and the
-// reciprocals may be approximate here.
-__device__ __forceinline__ void polar_scaled_step(const double X[3][3], const double C[3][3], double det, double nx,
-                                                  double nc, double Q[3][3]) {
-  const double g = 0.5 * __builtin_amdgcn_rsq(__builtin_amdgcn_rsq(nc * __builtin_amdgcn_rcp(nx)) * fabs(det));
-  const double w = 0.25 * __builtin_amdgcn_rcp(g * det);
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) Q[i][j] = g * X[i][j] + w * C[i][j];
-}
-
-// What the symmetric-Dirichlet local step takes from the SVD J = U diag(s) V^T, without an SVD.
-// With the left polar decomposition J = S Q (S = U diag(s) U^T, Q = U V^T) and T = S^-1:
-//   W^2 = U diag((s + 1)(s^2 + 1) / s^3) U^T = I + T + T^2 + T^3      (slim_m.cpp:337-353)
-//   R   = Q                                                          (det J > 0)
-//   dE/dJ = 2 (J - J^-T J^-1 J^-T) = 2 (S - T^3) Q
-// Q comes from Newton's iteration X <- (g X + X^-T / g) / 2, scaled by g = (|X^-1| / |X|)^(1/2)
-// in its first two steps (Higham's Frobenius scaling); it converges quadratically, so a step
-// that moved X by d leaves an error of about d^2 / 2 and the loop ends at d^2 < 4e-16: four to
-// six steps of some 80 operations, against up to 12 Jacobi sweeps of three rotations with a
-// division and three square roots each.
-//
-// sg = -1: J's columns come in an order that mirrors it (sg det J is the orientation); W2 and T3
-// do not see that, and Q is R with its columns in the same order.
-//
-// Returns false, leaving the outputs unset, where the SVD has to decide: J inverted or singular,
-// |J| |J^-1| above 1e3 (T and its powers then lose more digits than the singular values do), or
-// a singular value that may lie within the reference's band |s - 1| < 1e-8 where it sets its
-// weight to 1, unless all three do (an undeformed tet), which is W = I exactly. With D = S - I
-// the eigenvalue of D nearest 0 is at least |det D| / |adj D|; D carries an absolute error of a
-// few 1e-16, so a bound above 2e-8 keeps every singular value out of the band.
-// W2: xx, yy, zz, xy, xz, yz of W^2. T3 (T^3, the same order).
-__device__ __forceinline__ bool sd_polar(const double J[3][3], double sg, double Q[3][3], double W2[6], double T3[6]) {
-  double C[3][3];
-  cofactor3(J, C);
-  const double det = J[0][0] * C[0][0] + J[0][1] * C[0][1] + J[0][2] * C[0][2];
-  {
-    const double nj = norm2_3(J), nc = norm2_3(C);
-    if (!(sg * det > 0.0 && nj * nc < 1e6 * (det * det))) return false;
-    polar_scaled_step(J, C, det, nj, nc, Q);
-  }
-  cofactor3(Q, C);
-  polar_scaled_step(Q, C, Q[0][0] * C[0][0] + Q[0][1] * C[0][1] + Q[0][2] * C[0][2], norm2_3(Q), norm2_3(C), Q);
-  double d2 = 1.0;
-#pragma unroll 1
-  for (int it = 0; it < 12 && d2 > 4e-16; ++it) {
-    cofactor3(Q, C);
-    const double w = 0.5 * fast_rcp(Q[0][0] * C[0][0] + Q[0][1] * C[0][1] + Q[0][2] * C[0][2]);
-    d2 = 0.0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double m = w * C[i][j] - 0.5 * Q[i][j];
-        d2 += m * m;
-        Q[i][j] += m;
-      }
-  }
-  // D = S - I with S = J Q^T, and its adjugate
-  const double D[6] = {J[0][0] * Q[0][0] + J[0][1] * Q[0][1] + J[0][2] * Q[0][2] - 1.0,
-                       J[1][0] * Q[1][0] + J[1][1] * Q[1][1] + J[1][2] * Q[1][2] - 1.0,
-                       J[2][0] * Q[2][0] + J[2][1] * Q[2][1] + J[2][2] * Q[2][2] - 1.0,
-                       J[0][0] * Q[1][0] + J[0][1] * Q[1][1] + J[0][2] * Q[1][2],
-                       J[0][0] * Q[2][0] + J[0][1] * Q[2][1] + J[0][2] * Q[2][2],
-                       J[1][0] * Q[2][0] + J[1][1] * Q[2][1] + J[1][2] * Q[2][2]};
-  const double n2 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2] + 2.0 * (D[3] * D[3] + D[4] * D[4] + D[5] * D[5]);
-  if (n2 < 0.8e-16) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) W2[k] = k < 3 ? 1.0 : 0.0;
-  } else {
-    const double a00 = D[1] * D[2] - D[5] * D[5], a11 = D[0] * D[2] - D[4] * D[4], a22 = D[0] * D[1] - D[3] * D[3];
-    const double a01 = D[4] * D[5] - D[3] * D[2], a02 = D[3] * D[5] - D[4] * D[1], a12 = D[3] * D[4] - D[5] * D[0];
-    const double dd = D[0] * a00 + D[3] * a01 + D[4] * a02;
-    const double na = a00 * a00 + a11 * a11 + a22 * a22 + 2.0 * (a01 * a01 + a02 * a02 + a12 * a12);
-    if (!(d2 <= 4e-16 && dd * dd > 4e-16 * na)) return false;
-  }
-  // T = Q J^-1 = Q cof(J)^T / det J, symmetric
-  cofactor3(J, C);
-  const double id = fast_rcp(det);
-  const double T[6] = {id * (Q[0][0] * C[0][0] + Q[0][1] * C[0][1] + Q[0][2] * C[0][2]),
-                       id * (Q[1][0] * C[1][0] + Q[1][1] * C[1][1] + Q[1][2] * C[1][2]),
-                       id * (Q[2][0] * C[2][0] + Q[2][1] * C[2][1] + Q[2][2] * C[2][2]),
-                       id * (Q[0][0] * C[1][0] + Q[0][1] * C[1][1] + Q[0][2] * C[1][2]),
-                       id * (Q[0][0] * C[2][0] + Q[0][1] * C[2][1] + Q[0][2] * C[2][2]),
-                       id * (Q[1][0] * C[2][0] + Q[1][1] * C[2][1] + Q[1][2] * C[2][2])};
-  const double P[6] = {T[0] * T[0] + T[3] * T[3] + T[4] * T[4], T[3] * T[3] + T[1] * T[1] + T[5] * T[5],
-                       T[4] * T[4] + T[5] * T[5] + T[2] * T[2], T[0] * T[3] + T[3] * T[1] + T[4] * T[5],
-                       T[0] * T[4] + T[3] * T[5] + T[4] * T[2], T[3] * T[4] + T[1] * T[5] + T[5] * T[2]};
-  T3[0] = T[0] * P[0] + T[3] * P[3] + T[4] * P[4];
-  T3[1] = T[3] * P[3] + T[1] * P[1] + T[5] * P[5];
-  T3[2] = T[4] * P[4] + T[5] * P[5] + T[2] * P[2];
-  T3[3] = T[0] * P[3] + T[3] * P[1] + T[4] * P[5];
-  T3[4] = T[0] * P[4] + T[3] * P[5] + T[4] * P[2];
-  T3[5] = T[3] * P[4] + T[1] * P[5] + T[5] * P[2];
-  if (n2 >= 0.8e-16) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) W2[k] = T[k] + P[k] + T3[k] + (k < 3 ? 1.0 : 0.0);
-  }
-  return true;
-}
-
-// The same from the SVD, for the tets that sd_polar leaves to it: the weights
-// m^2 = (s - s^-3) / (s - 1) in the form that does not cancel at s = 1, and polar_svd's R (a
-// reflection is removed by negating V's last column).
-__device__ __forceinline__ void sd_svd(const double J[3][3], double W2[6], double R[3][3]) {
-  double U[3][3], s[3], V[3][3], m2[3];
-  svd3(J, U, s, V);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const double is = 1.0 / s[i];
-    m2[i] = fabs(s[i] - 1.0) < 1e-8 ? 1.0 : (s[i] + 1.0) * (s[i] * s[i] + 1.0) * is * is * is;
-  }
-  constexpr int r[6] = {0, 1, 2, 0, 0, 1}, c[6] = {0, 1, 2, 1, 2, 2};
-#pragma unroll
-  for (int k = 0; k < 6; ++k)
-    W2[k] = U[r[k]][0] * m2[0] * U[c[k]][0] + U[r[k]][1] * m2[1] * U[c[k]][1] + U[r[k]][2] * m2[2] * U[c[k]][2];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) R[i][j] = U[i][0] * V[j][0] + U[i][1] * V[j][1] + U[i][2] * V[j][2];
-  if (det3(R) < 0.0) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) R[i][j] = U[i][0] * V[j][0] + U[i][1] * V[j][1] - U[i][2] * V[j][2];
-  }
-}
-
 // Symmetric-Dirichlet SLIM weight matrix for the FP32 path: W = U diag(m) U^T with
 // m^2 = (s - s^-3)/(s - 1) evaluated as (s + 1)(s^2 + 1)/s^3 (the same function without the
 // cancellation at s -> 1 that FP32 cannot afford), and m = 1 where |s - 1| < 1e-8 as in

@@ -580,8 +580,6 @@ __device__ __forceinline__ void rotate_rings(T a[8][N]) {
 // Local step: per tet SVD -> W, R (slim_m.cpp:236-377); stores K = M W^T W (scaled by
 // invs^2 for the cube operator) and scatters the rhs A^T M (W R) (buildRhs, :1044-1092) and
 // the Jacobi diagonal of A^T M A (the DiagonalPreconditioner of the CG).
-// SD: the symmetric Dirichlet energy, whose weights need no SVD (sd_polar)
-template <bool SD>
 struct LocalStepOp {
   RefOp ro; int nV, nH; const int* conn; const double* X; double* K;
   int energy; double M, exp_f, prox;
@@ -598,21 +596,12 @@ struct LocalStepOp {
 #pragma unroll
       for (int d = 0; d < 3; ++d) E[d][k] = p[tc[k + 1]][d] - p[T0][d];
     matmul3(E, B, J);
+    slim_weights(J, energy, exp_f, W, R);
     double Kt[3][3];  // M W^T W
-    if constexpr (SD) {
-      double W2[6], cube[6];
-      if (!sd_polar(J, 1.0, R, W2, cube)) sd_svd(J, W2, R);
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) Kt[i][j] = M * W2[i == j ? i : i + j + 2];
-    } else {
-      slim_weights(J, energy, exp_f, W, R);
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) Kt[i][j] = M * (W[0][i] * W[0][j] + W[1][i] * W[1][j] + W[2][i] * W[2][j]);
-    }
+      for (int j = 0; j < 3; ++j) Kt[i][j] = M * (W[0][i] * W[0][j] + W[1][i] * W[1][j] + W[2][i] * W[2][j]);
     double s2 = 1.0;
     if (ro.mode == REF_CUBE) { double s = ro.invs[(size_t)c * nH + h]; s2 = s * s; }
     const double ks[6] = {Kt[0][0], Kt[1][1], Kt[2][2], Kt[0][1], Kt[0][2], Kt[1][2]};
@@ -620,9 +609,7 @@ struct LocalStepOp {
     for (int j = 0; j < 6; ++j) K[k_at<double>(c * 6 + j, h, nH)] = ks[j] * s2;
     // rhs: (W^T M W R) scattered through B
     double Z[3][3];
-    if constexpr (SD) {
-      matmul3(Kt, R, Z);
-    } else {
+    {
       double F[3][3];
       matmul3(W, R, F);
 #pragma unroll
@@ -711,132 +698,8 @@ struct LocalStepOp {
 // the FP64 local step needs all 256 registers on its own (one wave per SIMD); two waves per
 // SIMD hide its FP64 latency better than the registers it then spills cost (125 spilled
 // values: 2.13 ms against 2.63 ms per pass on the 1.1M-hex octree torus)
-template <bool SD>
-struct TileWaves<LocalStepOp<SD>> {
-  static constexpr int value = 2;
-};
-
-// Exchanges the two rings of a per-hex corner array (corner i and the one above it)
-template <class T, int N>
-__device__ __forceinline__ void swap_rings(T a[8][N]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int d = 0; d < N; ++d) {
-      const T b = a[i][d];
-      a[i][d] = a[i + 4][d];
-      a[i + 4][d] = b;
-    }
-}
-
-// The symmetric-Dirichlet local step on cube references. There the reference operator of a
-// corner tet is invs times a rotation of the axes, which neither the weights nor the forces
-// see: with J = invs E (E the three edges), K = invs^2 M W^2, the force on edge k is column k of
-// M invs W^2 Q and every edge adds K's diagonal at both of its ends. So no operator B is formed
-// or multiplied. The four tets of a ring are unrolled (compile-time rows, no turning of the
-// corner arrays), and the upper ring runs the same code on exchanged rings: there corner c's
-// neighbours {c - 1, c + 1, c - 4} come as {c - 1, c - 4, c + 1}, a mirrored order (sg = -1).
-struct LocalStepCubeOp : LocalStepOp<true> {
-  __device__ __forceinline__ void store_K(int h, int c, const double ks[6]) const {
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      *reinterpret_cast<double2*>(K + k_at<double>(c * 6 + 2 * j, h, nH)) = make_double2(ks[2 * j], ks[2 * j + 1]);
-  }
-  // false: nothing added, the tet is left to svd_tet
-  template <int R0>
-  __device__ __forceinline__ bool cube_tet(int h, int c, double sg, const double p[8][3], double out[8][6]) const {
-    constexpr int tc[3] = {(R0 + 3) & 3, R0 + 4, (R0 + 1) & 3};
-    const double s = ro.invs[(size_t)c * nH + h];
-    double J[3][3], W2[6], T3[6], Q[3][3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) J[d][k] = s * (p[tc[k]][d] - p[R0][d]);
-    if (!sd_polar(J, sg, Q, W2, T3)) return false;
-    const double ms = M * s, ms2 = ms * s;
-    double ks[6];
-#pragma unroll
-    for (int j = 0; j < 6; ++j) ks[j] = ms2 * W2[j];
-    store_K(h, c, ks);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const double f[3] = {ms * (W2[0] * Q[0][k] + W2[3] * Q[1][k] + W2[4] * Q[2][k]),
-                           ms * (W2[3] * Q[0][k] + W2[1] * Q[1][k] + W2[5] * Q[2][k]),
-                           ms * (W2[4] * Q[0][k] + W2[5] * Q[1][k] + W2[2] * Q[2][k])};
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        out[tc[k]][d] += f[d];
-        out[R0][d] -= f[d];
-        out[tc[k]][3 + d] += ks[d];
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) out[R0][3 + d] += 3.0 * ks[d];
-    return true;
-  }
-  // corner tet c by its SVD. Rare: its corners are loaded again and its rows picked by selects.
-  __device__ __forceinline__ void svd_tet(int h, int c, double out[8][6]) const {
-    const double s = ro.invs[(size_t)c * nH + h];
-    double J[3][3], W2[6], R[3][3], x0[3];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int v = conn[(size_t)kHexTet[c][k] * nH + h];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double x = X[(size_t)d * nV + v];
-        if (k == 0) x0[d] = x;
-        else J[d][k - 1] = s * (x - x0[d]);
-      }
-    }
-    sd_svd(J, W2, R);
-    const double ms = M * s, ms2 = ms * s;
-    double ks[6], k3[3];
-#pragma unroll
-    for (int j = 0; j < 6; ++j) ks[j] = ms2 * W2[j];
-    store_K(h, c, ks);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const double f[3] = {ms * (W2[0] * R[0][k] + W2[3] * R[1][k] + W2[4] * R[2][k]),
-                           ms * (W2[3] * R[0][k] + W2[1] * R[1][k] + W2[5] * R[2][k]),
-                           ms * (W2[4] * R[0][k] + W2[5] * R[1][k] + W2[2] * R[2][k])};
-      const double mf[3] = {-f[0], -f[1], -f[2]};
-      add_row<0, 3>(out, kHexTet[c][k + 1], f);
-      add_row<0, 3>(out, kHexTet[c][0], mf);
-      add_row<3, 3>(out, kHexTet[c][k + 1], ks);
-      k3[k] = 3.0 * ks[k];
-    }
-    add_row<3, 3>(out, kHexTet[c][0], k3);
-  }
-  __device__ double hex(int h, double out[8][6]) const {
-    unsigned left = 0;
-    {
-      int vid[8];
-      double p[8][3];
-      gather8(X, nV, conn, nH, h, vid, p);
-#pragma unroll 1
-      for (int c = 0; c < 8; c += 4) {
-        const double sg = c == 0 ? 1.0 : -1.0;
-        left |= (unsigned)!cube_tet<0>(h, c, sg, p, out) << c;
-        left |= (unsigned)!cube_tet<1>(h, c + 1, sg, p, out) << (c + 1);
-        left |= (unsigned)!cube_tet<2>(h, c + 2, sg, p, out) << (c + 2);
-        left |= (unsigned)!cube_tet<3>(h, c + 3, sg, p, out) << (c + 3);
-        swap_rings(p);
-        swap_rings(out);
-      }
-    }
-#pragma unroll 1
-    for (int c = 0; c < 8; ++c)
-      if ((left >> c) & 1) svd_tet(h, c, out);
-    return 0.0;
-  }
-};
-
-// VALU-bound (FP64): 2257 us with the SVD, 374 us in this form per pass on the 1.1M-hex octree
-// torus (567 and 82 us on the 64^3 grid); 254 registers, so two waves per SIMD without spills.
-// The tets left to the SVD run after the unrolled ones instead of in a branch or a call inside
-// them: their registers would make every tet spill (729 us with a call).
 template <>
-struct TileWaves<LocalStepCubeOp> {
+struct TileWaves<LocalStepOp> {
   static constexpr int value = 2;
 };
 
@@ -2576,16 +2439,8 @@ void launch_ref_general(const double* X, int nV, const int* conn, int nH, const 
 void launch_local_step(const TileMesh& tm, const RefOp& ro, const double* X, double* K, int energy, double M,
                        double exp_f, double prox, const SoftDev& sd, double* rhs, double* invd, double* halo,
                        hipStream_t st) {
-  if (energy == E_SYMMETRIC_DIRICHLET && ro.mode == REF_CUBE) {
-    LocalStepCubeOp op{{ro, tm.nV, tm.nH, tm.conn, X, K, energy, M, exp_f, prox, sd, rhs, invd}};
-    launch_scatter<double, 6>(tm, op, halo, nullptr, nullptr, st);
-  } else if (energy == E_SYMMETRIC_DIRICHLET) {
-    LocalStepOp<true> op{ro, tm.nV, tm.nH, tm.conn, X, K, energy, M, exp_f, prox, sd, rhs, invd};
-    launch_scatter<double, 6>(tm, op, halo, nullptr, nullptr, st);
-  } else {
-    LocalStepOp<false> op{ro, tm.nV, tm.nH, tm.conn, X, K, energy, M, exp_f, prox, sd, rhs, invd};
-    launch_scatter<double, 6>(tm, op, halo, nullptr, nullptr, st);
-  }
+  LocalStepOp op{ro, tm.nV, tm.nH, tm.conn, X, K, energy, M, exp_f, prox, sd, rhs, invd};
+  launch_scatter<double, 6>(tm, op, halo, nullptr, nullptr, st);
 }
 
 void launch_adj_local32(const TileMesh& tm, const RefOp& ro, const double* X, float* K, double M, double prox,

@@ -1,6 +1,6 @@
 """The symmetric-Dirichlet local step against its definition, tet by tet: single hexes whose
-corner tets all have one known Jacobian U diag(s) V^T, over the singular values where the polar
-form hands over to the SVD (undeformed, inside and just outside the band |s - 1| < 1e-8,
+corner tets all have one known Jacobian U diag(s) V^T, over singular values where the weights
+change form or lose digits (undeformed, inside and just outside the band |s - 1| < 1e-8,
 ill-conditioned, inverted) and on both reference operators (cube, general)."""
 import numpy as np
 import pytest
@@ -26,15 +26,14 @@ def weight2(s):
 
 
 @pytest.mark.parametrize("cube", [True, False])
-@pytest.mark.parametrize("precision", [64])
-def test_weights_rhs_and_diagonal(cube, precision):
+def test_weights_rhs_and_diagonal(cube):
     from pyhexopt import capi, meshgen as mg
     rng = np.random.default_rng(11)
     nH = len(SIGMA) * 25                       # 325 hexes: several tiles, the last one partly filled
     box = mg.HEX_CORNERS - 0.5
     V = np.tile(box, (nH, 1))
     H = np.arange(8 * nH, dtype=np.int32).reshape(nH, 8)
-    A, want, rot, kappa = [], [], [], []
+    A, want, rot, kappa, near = [], [], [], [], []
     for h in range(nH):
         s = np.array(SIGMA[h % len(SIGMA)], dtype=float)
         U, W = rotation(rng), rotation(rng)
@@ -44,23 +43,24 @@ def test_weights_rhs_and_diagonal(cube, precision):
         # the closest rotation: an inverted tet's smallest direction is flipped back
         rot.append(U @ W.T)
         kappa.append(a.max() / a.min())
-    A, want, rot, kappa = np.array(A), np.array(want), np.array(rot), np.array(kappa)
+        # distance from 1 of the singular value nearest to it outside the band
+        near.append(min([abs(x - 1) for x in a if abs(x - 1) >= 1e-8], default=np.inf))
+    A, want, rot, kappa, near = (np.array(x) for x in (A, want, rot, kappa, near))
     X = np.einsum("hij,hkj->hki", A, V.reshape(nH, 8, 3)).reshape(-1, 3)
     h = capi.HexOpt(V, H)
     h.reference(cube=cube)
     h.set_positions(capi.CURRENT, X)
-    K = h.debug_operator(precision)
+    K = h.debug_operator()
     # a unit cube's corner tets have reference factor 1, so K is W^2 (and a general reference
     # operator turns the axes of J's right side only, which W does not see)
     got = K[:, :, [0, 3, 4, 3, 1, 5, 4, 5, 2]].reshape(nH, 8, 3, 3)
     scale = np.abs(want).max(axis=(1, 2))
     err = np.abs(got - want[:, None]).max(axis=(1, 2, 3)) / scale
-    # J's entries carry an error of a few eps |J|, which moves T = S^-1 by that times kappa and its
-    # cube by three times as much; the stored FP32 blocks add half an ulp
-    tol = 60 * EPS * kappa + (0 if precision == 64 else 1e-7)
+    # J's entries carry an error of a few eps |J|, which moves 1/s by that times kappa and its cube by
+    # three times as much; the reference's form of the weight, (s - s^-3) / (s - 1), rounds its
+    # numerator to a few eps and divides it by s - 1
+    tol = 60 * EPS * kappa + 4 * EPS / near
     assert (err < tol).all(), (err / tol).max()
-    if precision == 32:
-        return
     prox = 1e-5
     rhs, invd, _ = h.debug_system(X.T.reshape(-1))
     rhs, diag = rhs.reshape(3, -1).T.reshape(nH, 8, 3), 1.0 / invd.reshape(3, -1).T.reshape(nH, 8, 3)
