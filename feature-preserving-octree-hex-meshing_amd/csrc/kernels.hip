@@ -1460,9 +1460,9 @@ __device__ __forceinline__ void pipe_fetch(const TileMesh& tm, const float* __re
 // us, on 262,144 27.3 -> 25.0). A compact tile of 256 hexes has about 400 of them, so two rounds of the
 // block are fetched ahead; what a ragged tile has beyond them is loaded where it is staged.
 constexpr int kAhead = 2;
-template <class T, class TILE>
-__device__ __forceinline__ void pipe_gather(const TILE& P, int nV, const T* __restrict__ z,
-                                            const T* __restrict__ pprev, bool prev, T zr[kAhead][3], T pr[kAhead][3]) {
+__device__ __forceinline__ void pipe_gather(const PipeTile& P, int nV, const float* __restrict__ z,
+                                            const float* __restrict__ pprev, float zr[kAhead][3],
+                                            float pr[kAhead][3]) {
 #pragma unroll
   for (int j = 0; j < kAhead; ++j) {
     if ((int)threadIdx.x + j * kTileHex < P.nlv) {
@@ -1470,7 +1470,7 @@ __device__ __forceinline__ void pipe_gather(const TILE& P, int nV, const T* __re
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
         zr[j][d] = z[(size_t)d * nV + g];
-        pr[j][d] = prev ? pprev[(size_t)d * nV + g] : T(0);
+        pr[j][d] = pprev[(size_t)d * nV + g];
       }
     }
   }
@@ -1504,7 +1504,7 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_pipe_kernel(TileMesh tm, 
   float zr[kAhead][3], pr[kAhead][3];
   if (tile < tend) {
     pipe_fetch(tm, K, tile, P);
-    pipe_gather(P, nV, z, pprev, true, zr, pr);
+    pipe_gather(P, nV, z, pprev, zr, pr);
   }
   // (the first tile's loads are in flight while the beta step is formed)
   float beta;
@@ -1590,7 +1590,7 @@ __global__ __launch_bounds__(kTileHex) void cg32_apply_pipe_kernel(TileMesh tm, 
         halo[sl[j]] = acc[lv];
       }
     }
-    if (tile < tend) pipe_gather(P, nV, z, pprev, true, zr, pr);
+    if (tile < tend) pipe_gather(P, nV, z, pprev, zr, pr);
     // the next tile's staging overwrites sp and acc
     __syncthreads();
   }
