@@ -58,9 +58,9 @@ __host__ __device__ inline int stack_frames(int depth) {
 void launch_closest(const SurfaceDev& s, int nq, const double* P, int soa, int stride, const int* ids, double* S, int* I,
                     double* C, double* N, double* sqrD, int* status, hipStream_t st, const int* order = nullptr);
 
-// Lanes of a wave that take a query each, for nq queries in a launch: a block of kBvhBlock
-// threads takes closest_lanes(nq) * kBvhBlock / 64 of them.
-int closest_lanes(int nq);
+// Lanes of a wave that take a query each, for nq queries of nseg segments in a launch: a block of
+// kBvhBlock threads takes closest_lanes(nq, nseg) * kBvhBlock / 64 queries of one segment.
+int closest_lanes(int nq, int nseg);
 
 // Several surfaces in one launch: segment j's queries are order[q0 .. q0 + n) against surface
 // s, taken by blocks block0 .. block0 + ceil(n / a block's queries) (segments in increasing block0,

@@ -429,16 +429,30 @@ void launch_metro_ep(const SurfaceDev& s, const double* ep, int nq, const double
 
 // A walk is a chain of some 150 dependent steps for the longest of a wave's queries, and a wave
 // runs a leaf and an inner step in every round its lanes disagree. Few queries leave most of the
-// device idle whatever is done, so they are spread over more waves of fewer lanes: 488 queries on
-// 20,480 triangles take 257 us with 64 lanes, 234 with 32, 211 with 16, 191 with 8; 10,088
-// queries 248, 231, 272 and 284, and 411,080 queries 253, 321, 457 and 762.
-int closest_lanes(int nq) { return nq <= 2048 ? 8 : 64; }
+// device idle whatever is done, so they are spread over more waves of fewer lanes, as many as keep
+// to one block on each of the 256 CUs: a second block on a CU costs more than fewer lanes gain.
+// us per refresh of the planes of a grid's boundary on 20,480 triangles:
+//   queries    488  2,402  4,058  6,146  7,778  10,088  15,002  24,578
+//    8 lanes   192    196    201    249    248     299     345     375
+//   16         214    216    217    222    220     277     281     281
+//   32         239    237    236    239    234     233     232     264
+//   64         264    256    253    255    252     250     247     247
+// (the same order on 1,280 triangles and with random queries). Segments of a launch may each add a
+// block that is not full.
+int closest_lanes(int nq, int nseg) {
+  constexpr int kCUs = 256;
+  for (int lanes = 8; lanes < 64; lanes *= 2) {
+    const int per_block = lanes * (kBvhBlock / 64);
+    if ((nq - 1) / per_block + nseg <= kCUs) return lanes;
+  }
+  return 64;
+}
 
 void launch_closest(const SurfaceDev& s, int nq, const double* P, int soa, int stride, const int* ids, double* S, int* I,
                     double* C, double* N, double* sqrD, int* status, hipStream_t st, const int* order) {
   if (nq <= 0) return;
   const size_t lds = (size_t)stack_frames(s.depth) * kBvhBlock * sizeof(uint2);
-  const int lanes = closest_lanes(nq), per_block = lanes * (kBvhBlock / 64);
+  const int lanes = closest_lanes(nq, 1), per_block = lanes * (kBvhBlock / 64);
   hipLaunchKernelGGL(closest_kernel, dim3((nq + per_block - 1) / per_block), dim3(kBvhBlock), lds, st, s,
                      (const PatchSeg*)nullptr, 0, lanes, nq, P, soa, stride, ids, order, S, I, C, N, sqrD, status);
 }

@@ -1339,7 +1339,7 @@ int hexopt_project_patches(hexopt_ctx* c, int npatch, hexopt_surface* const* pat
   // all patches in one launch: normal_T = pseudonormal N, dis_T = N . closest point
   std::vector<PatchSeg> segs;
   int nblocks = 0, max_depth = 1;
-  const int lanes = closest_lanes(nT), per_block = lanes * (kBvhBlock / 64);
+  const int lanes = closest_lanes(nT, npatch), per_block = lanes * (kBvhBlock / 64);
   for (int p = 0; p < npatch; ++p) {
     const int n = c->patch_off[p + 1] - c->patch_off[p];
     if (n == 0) continue;

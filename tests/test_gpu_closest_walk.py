@@ -13,13 +13,13 @@ def same(a, b):
     return all(np.array_equal(x, y) for x, y in zip(a, b))
 
 
-@pytest.mark.parametrize("nq", [1, 7, 16, 17, 2047, 2048, 2049, 4096])
+@pytest.mark.parametrize("nq", [1, 7, 16, 17, 2047, 2048, 2049, 4095, 4096, 4097, 8192, 8193, 16384, 16385])
 def test_number_of_queries(nq):
     from pyhexopt import capi, meshgen as mg
     SV, SF = mg.superellipsoid(3)
     s = capi.Surface(SV, SF)
     rng = np.random.default_rng(1)
-    P = rng.uniform(-1.2, 1.2, size=(4096, 3))
+    P = rng.uniform(-1.2, 1.2, size=(16385, 3))
     P[::5] = SV[rng.integers(0, SV.shape[0], size=P[::5].shape[0])]        # on vertices: many faces tie
     all_ = s.closest(P)
     part = s.closest(P[:nq])
