@@ -1797,6 +1797,7 @@ static int adj_common(hexopt_ctx* c, int precision, const void* X, const void* v
 int hexopt_energy_grad(hexopt_ctx* c, const hexopt_params* prm, int precision, const void* X, const double* aL, void* G) {
   if (!c || !prm || !X || !G || (precision != 32 && precision != 64)) return HEXOPT_EINVAL;
   if (c->ref_mode < 0) return fail(c, HEXOPT_EINVAL, "hexopt_reference has not been called");
+  const OnDevice on(c->device);
   if (prm->energy != HEXOPT_SYMMETRIC_DIRICHLET) return fail(c, HEXOPT_EUNSUPPORTED, "adjoint supports SYMMETRIC_DIRICHLET");
   int rc = adj_common(c, precision, X, nullptr);
   if (rc) return rc;
@@ -1814,6 +1815,7 @@ int hexopt_energy_grad(hexopt_ctx* c, const hexopt_params* prm, int precision, c
 int hexopt_hvp(hexopt_ctx* c, const hexopt_params* prm, int precision, const void* X, const void* v, void* Hv) {
   if (!c || !prm || !X || !v || !Hv || (precision != 32 && precision != 64)) return HEXOPT_EINVAL;
   if (c->ref_mode < 0) return fail(c, HEXOPT_EINVAL, "hexopt_reference has not been called");
+  const OnDevice on(c->device);
   if (prm->energy != HEXOPT_SYMMETRIC_DIRICHLET) return fail(c, HEXOPT_EUNSUPPORTED, "adjoint supports SYMMETRIC_DIRICHLET");
   int rc = adj_common(c, precision, X, v);
   if (rc) return rc;
