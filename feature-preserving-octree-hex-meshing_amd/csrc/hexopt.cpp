@@ -1556,6 +1556,14 @@ int hexopt_octree_copy(const hexopt_octree* o, int32_t* leaves, int32_t* nodes, 
   const OnDevice on(o->device);
   std::string err;
   if (octree_copy(*o->dev, o->r, leaves, nodes, V, H, err)) return HEXOPT_OK;
+  // no copy may still write into the caller's memory, and a caller that does not look at the code
+  // finds zeros instead of what its memory held
+  (void)hipStreamSynchronize(hipStreamPerThread);
+  const size_t n = (size_t)o->r.leaves, m = (size_t)o->r.nodes;
+  if (leaves) std::fill_n(leaves, n * 4, 0);
+  if (nodes) std::fill_n(nodes, m * 3, 0);
+  if (V) std::fill_n(V, m * 3, 0.0);
+  if (H) std::fill_n(H, n * 8, 0);
   g_octree_error = err;
   return HEXOPT_EHIP;
 }

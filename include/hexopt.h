@@ -305,7 +305,8 @@ int hexopt_octree_refine(hexopt_octree* o, hexopt_surface* s, int stop_extent, i
  * (mesh_transform + origin + voxel_size * position, octree_mesh's mo.V) and H[n][8] (node
  * ids of each leaf's corners in the reference's corner order, octree_mesh's mo.Hs); any may
  * be NULL. The results stay on the octree's device until it is destroyed or refined and are
- * copied from there: HEXOPT_EHIP if the device fails (hexopt_octree_error() says why). */
+ * copied from there: HEXOPT_EHIP, and zeros in the arrays, if the device fails
+ * (hexopt_octree_error() says why). */
 int hexopt_octree_copy(const hexopt_octree* o, int32_t* leaves, int32_t* nodes, double* V, int32_t* H);
 
 /* ---- feature-curve projection (LINE branch of dirty_graph_projection,
