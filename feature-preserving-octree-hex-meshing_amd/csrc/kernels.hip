@@ -1977,8 +1977,8 @@ __device__ __forceinline__ double first_step(double tmin) {
 // tmin, two rows of blocks: the first the energies of the start (part), the second those of the
 // line search's first step, which follows from *tmin (part1). They go in one launch, with the step
 // formed here, because a search almost always ends at its first step: the host then reads bound
-// and energies once instead of twice and three launches go. One FP64 iteration on 729 hexes
-// 745 -> 632 us, with the other read-backs joined too. (Both energies in one thread needs 344
+// and energies once instead of twice and three launches go. One FP32 iteration on 729 hexes
+// 675 -> 561 us, with the other read-backs joined too. (Both energies in one thread needs 344
 // registers instead of 124, and 1.1M hexes then lose 150 us.)
 template <class T, bool DIFF, class DT>
 __global__ __launch_bounds__(256) void energy_kernel(RefOp ro, const double* cur, const DT* dst, double step, int nV, const int* conn,
